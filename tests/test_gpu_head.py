@@ -126,3 +126,23 @@ def test_timestamp_head_ragged_width(ctx, pkg, orc):
     top2 = np.sort(want_l, axis=1)[:, -2:]
     sure = top2[:, 1] - top2[:, 0] > 2 * bound.max(axis=1)
     assert np.array_equal(cls[sure], want_c[sure])
+
+
+@pytest.mark.parametrize("rows,labels,n", [(1, 33, 4), (32, 64, 68), (33, 4100, 192), (65, 5000, 1028), (97, 8200, 72)])
+def test_timestamp_head_tile_edges(ctx, pkg, rows, labels, n):
+    """The matrix-core logits at the edges of their tiles (32 rows, 32 or 64
+    labels, 64-deep slabs, fewer slabs than the ring): against 64 bits, within
+    (n + 64) f32 ulps of sum |normed| |score| (n products and sums, and the
+    norm's own); classes are the first maximum of the logits themselves."""
+    rng = np.random.default_rng(rows * labels + n)
+    h = (rng.standard_normal((rows + 3, n)) * 3).astype(np.float16)
+    w = (1.0 + 0.3 * rng.standard_normal(n)).astype(np.float32)
+    score = (0.05 * rng.standard_normal((labels, n))).astype(np.float32)
+    score[labels // 2:] = score[: labels - labels // 2]  # every maximum twice: the first one counts
+    pos = rng.permutation(rows + 3)[:rows].astype(np.int32)
+    logits, cls = _gpu_head(ctx, pkg, F16, h.view(np.uint16), pos, w, 1e-6, score)
+    x = h[pos].astype(np.float64) * w
+    y = x / np.sqrt((x ** 2).mean(axis=1, keepdims=True) + 1e-6)
+    bound = (n + 64) * 2.0 ** -24 * (np.abs(y) @ np.abs(score.astype(np.float64)).T)
+    assert (np.abs(logits - y @ score.astype(np.float64).T) <= bound).all()
+    assert np.array_equal(cls, logits.argmax(axis=1))
