@@ -6,11 +6,25 @@
 // arithmetic it must match is the CPU twin, src/cpu_decoder.rs:324-411: f32
 // scores q.k / sqrt(hd), softmax in f32, out = round(sum_t p_t v_t).
 //
-// Block = one kv head x a tile of 64 query rows x its REP q heads; waves:
-// NS = 2 key splits x REP heads x 2 row groups of 32.  Split s takes the key
-// blocks kb = s, s + 2, ... (64 keys each) below the tile's causal bound, so
-// the long rows' key range is processed by two wave groups at once; the two
-// partial results merge through LDS at the end in a fixed order.
+// Block = one kv head x a tile of RG x 32 query rows x its REP q heads; waves:
+// NS key splits x REP heads x RG row groups of 32.  Split s takes the key
+// blocks kb = s, s + NS, ... (64 keys each) below the tile's causal bound, so
+// the long rows' key range is processed by NS wave groups at once; the partial
+// results merge through LDS at the end in a fixed order.  Two shapes of eight
+// waves (REP = 2):
+//  * RG = 2, NS = 2: each K / V tile feeds 64 rows.  Once the grid is a few
+//    blocks per CU, the stream and the phases per FLOP decide (4334 rows: 127
+//    us against 138 with the other shape).
+//  * RG = 1, NS = 4: twice the blocks and half the steps in a row, for grids
+//    that leave CUs idle, where the length of the longest block's chain of
+//    steps decides (a phase is ~1 us however few blocks run).  Its four
+//    groups hold one K and one V tile each (NB = 1: 128 KB), refilled during
+//    the VALU phase, longer than the L2 takes to answer; with two of each of
+//    half the keys a step's fixed costs double (1024 rows: 20.1 us).
+//    Measured, f16, RG = 2 -> RG = 1: 61 rows 8.3 -> 7.1 us, 323 rows 12.9 ->
+//    10.5, 1024 rows 25.2 -> 17.8, 2048 rows (256 blocks of 64) 42.6 -> 36.1,
+//    2200 rows (280) 46.0 -> 48.3; 771 rows from position 1536 with 16-bit
+//    probabilities 38.8 -> 24.6.  Hence the line at 256 blocks of 64 rows.
 //
 // Per key block, per wave (32 query rows):
 //  * S = K . Q^T on v_mfma_f32_32x32x16 (A = 32 keys x 16 d from LDS, B = the
@@ -32,8 +46,8 @@
 //    keys {16j+4h..+3, 16j+8+4h..+3} of slice j, so the transposed V cache
 //    stores each aligned group of 16 keys in the order 0-3, 8-11, 4-7, 12-15
 //    (bits 2 and 3 of the key swapped): one 16-byte read per V fragment.
-//  * K and V tiles stream L2 -> LDS with buffer_load ... lds, double-buffered
-//    per split group; chunks are XOR-swizzled per row so the 32-row fragment
+//  * K and V tiles stream L2 -> LDS with buffer_load ... lds, NB buffers of
+//    each per split group; chunks are XOR-swizzled per row so the 32-row fragment
 //    reads hit distinct banks.
 #include <type_traits>
 
@@ -65,11 +79,9 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 #define QA_LDS __attribute__((address_space(3)))
 
-constexpr uint32_t OOB = 0x80000000u;
+constexpr uint32_t OOB = 0x80000000u;  // byte offset past every buffer's num_records
 constexpr int HD = 128;  // head dim
-constexpr int QT = 64;   // query rows per block
-constexpr int KB = 64;   // keys per block
-constexpr int NS = 2;    // key splits per block
+constexpr int KB = 64;   // keys per step
 constexpr float kLog2e = 1.44269504088896341f;
 // The running row max is raised only when a block's max exceeds it by more
 // than this (log2 units): probabilities then stay <= 2^kLazy and the output
@@ -148,6 +160,9 @@ struct AFmt<QA_BF16> {
   static constexpr float kPBias = 0.f;
 };
 
+// A value the caller knows to be equal in every lane, as a scalar register.
+__device__ __forceinline__ int wave_uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
   static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
@@ -171,20 +186,29 @@ __device__ __forceinline__ void exec_barrier() {
 __device__ __forceinline__ int kswz(int r) { return r & 15; }
 __device__ __forceinline__ int vswz(int d) { return (d >> 1) & 7; }
 
-template <int DT, int REP, int PS>
-__global__ void __launch_bounds__(NS * REP * 2 * 64) attention_kernel(const AttnParams p) {
-  constexpr int GW = REP * 2;        // waves per split group
-  constexpr int KTILE = KB * HD * 2;  // 16 KB
-  constexpr int VTILE = HD * KB * 2;  // 16 KB
+// RG row groups of 32 query rows per block, NS key splits, NB buffers of each
+// split's K and V tiles.
+template <int DT, int REP, int PS, int RG, int NS, int NB>
+__global__ void __launch_bounds__(NS * REP * RG * 64) attention_kernel(const AttnParams p) {
+  constexpr int QT = 32 * RG;          // query rows per block
+  constexpr int KT = KB / 32;          // 32-key score tiles per step
+  constexpr int GW = REP * RG;         // waves per split group
+  constexpr int VCH = KB / 8;          // 16-byte chunks per V tile row
+  constexpr int VR = 64 / VCH;         // V tile rows per DMA instruction
+  constexpr int KTILE = KB * HD * 2;
+  constexpr int VTILE = HD * KB * 2;
   constexpr int KI = KB * HD * 2 / 1024 / GW;  // K DMA instructions per wave per block
   constexpr int VI = HD * KB * 2 / 1024 / GW;  // V DMA instructions per wave per block
   constexpr int LPS = KI + VI;
-  static_assert(KI * GW * 4 == KB && VI * GW * 8 == HD, "DMA row coverage");
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[NS * 2 * (KTILE + VTILE)];
+  static_assert(KI * GW * 4 == KB && VI * GW * VR == HD, "DMA row coverage");
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[NS * NB * (KTILE + VTILE)];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int split = wave / GW, wg = wave % GW;
-  const int hh = wg / 2, rg = wg & 1;
+  const int hh = wg / RG, rg = wg % RG;
+  // Phase offset (see the phases below): a SIMD runs waves w and w + 4, so the
+  // upper half of the split groups runs one phase behind the lower half.
+  const int off = split / (NS / 2);
   const int fr = lane & 31, fh = lane >> 5;
 #ifdef QA_PHASE_STAMPS
   // s_memtime cycles by phase: prologue, MFMA, VALU, no work, barrier,
@@ -207,10 +231,10 @@ __global__ void __launch_bounds__(NS * REP * 2 * 64) attention_kernel(const Attn
   const int64_t kend = p.q0 + min(row0 + QT, p.rows);  // keys 0..kend-1 are visible
   const int nkb = (int)((kend + KB - 1) / KB);
 
-  // ---- LDS: per split group, K slots 0/1 then V slots 0/1 (16 KB each) ----
-  unsigned char* gsm = smem + split * 2 * (KTILE + VTILE);
-  auto kslot = [&](int it) { return gsm + (it & 1) * KTILE; };
-  auto vslot = [&](int it) { return gsm + 2 * KTILE + (it & 1) * VTILE; };
+  // ---- LDS: per split group, K slots 0/1 then V slots 0/1 ----
+  unsigned char* gsm = smem + split * NB * (KTILE + VTILE);
+  auto kslot = [&](int it) { return gsm + (it & (NB - 1)) * KTILE; };
+  auto vslot = [&](int it) { return gsm + NB * KTILE + (it & (NB - 1)) * VTILE; };
   // this group's steps: key blocks split, split + NS, ... below nkb
   const int nst = (nkb - split + NS - 1) / NS;
 
@@ -221,14 +245,14 @@ __global__ void __launch_bounds__(NS * REP * 2 * 64) attention_kernel(const Attn
       const_cast<uint16_t*>(kbase), (short)0, (int)(p.cap * HD * 2), 0x00020000);
   const __amdgpu_buffer_rsrc_t rsv = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint16_t*>(vbase), (short)0, (int)(p.cap * HD * 2), 0x00020000);
-  // Per-lane byte offsets of this wave's chunks at key block 0.  K
-  // instruction j fills key rows 4 (GW j + wg) + lane / 16 and V instruction j
-  // d rows 8 (GW j + wg) + lane / 8; with GW = 4 the K chunk swizzle (row & 15)
-  // and for any GW the V chunk swizzle ((d >> 1) & 7) are the same for every
-  // j, so instruction j's offset is the lane's offset at j = 0 plus a
-  // wave-uniform amount: one add per instruction.  K rows at or past cap lie
-  // past the buffer's num_records and read as zeros; a V column at or past cap
-  // would not (it lies inside the next d row), so those lanes get OOB.
+  // K instruction j fills key rows 4 (GW j + wg) + lane / 16 and V instruction
+  // j d rows VR (GW j + wg) + lane / VCH.  Over j the chunk swizzle of a lane's
+  // V rows stays the same, and that of its K rows (row & 15) does for GW = 4
+  // and alternates in bit 3 for GW = 2: an instruction's offset is the lane's
+  // offset at j = 0 (that bit toggled) plus a wave-uniform amount, one add.
+  // K rows at or past cap lie past the buffer's num_records and read as zeros;
+  // a V column at or past cap (the last block, cap % KB != 0) would not, as it
+  // lies inside the next d row, so those lanes get OOB.
   // (The lane offsets are recomputed at each refill, a few instructions, from
   // a copy of the lane index the compiler cannot hoist: kept live across the
   // loop they would push the kernel past its register budget.)
@@ -237,47 +261,40 @@ __global__ void __launch_bounds__(NS * REP * 2 * 64) attention_kernel(const Attn
     asm volatile("" : "+v"(l));
     return l;
   };
+  static_assert(GW * 4 % 16 == 0 || GW * 4 % 16 == 8, "K chunk swizzle over j");
+  static_assert(GW * VR % 16 == 0, "V chunk swizzle over j");
   auto issue_k = [&](int it) {
-    unsigned char* sk = kslot(it);
-    const int kb = split + NS * it;
+    unsigned char* sk = smem + wave_uniform((int)(kslot(it) - smem) + wg * 1024);
     const int l = lane_opaque(), rk = wg * 4 + (l >> 4);
     const uint32_t koff0 = (uint32_t)((rk * HD + (((l & 15) ^ kswz(rk)) << 3)) * 2);
+    const uint32_t kb0 = (uint32_t)(split + NS * it) * (KB * HD * 2);
 #pragma unroll
     for (int j = 0; j < KI; ++j) {
-      const int ins = j * GW + wg;
-      uint32_t off;
-      if constexpr (GW * 4 % 16 == 0) {
-        off = koff0 + (uint32_t)(((int64_t)kb * KB + 4 * GW * j) * HD * 2);
-      } else {
-        const int r = ins * 4 + (l >> 4);  // key row within the tile
-        const int64_t key = (int64_t)kb * KB + r;
-        off = key < p.cap ? (uint32_t)((key * HD + (((l & 15) ^ kswz(r)) << 3)) * 2) : OOB;
-      }
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsk, (QA_LDS void*)(sk + ins * 1024), 16, off, 0,
-                                               0, 0);
+      const uint32_t flip = GW * 4 * j % 16 * 16;  // bit 3 of the chunk
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsk, (QA_LDS void*)(sk + j * GW * 1024), 16,
+                                               (koff0 ^ flip) + kb0 + 4 * GW * j * HD * 2, 0, 0, 0);
     }
   };
   auto issue_v = [&](int it) {
-    unsigned char* sv = vslot(it);
-    const int kb = split + NS * it;
-    const int l = lane_opaque(), dv = wg * 8 + (l >> 3);
-    const int vc = ((l & 7) ^ vswz(dv)) << 3;
-    const uint32_t voff0 = (uint32_t)(((int64_t)dv * p.cap + vc) * 2);
-    const bool vin = (int64_t)kb * KB + vc < p.cap;
+    unsigned char* sv = smem + wave_uniform((int)(vslot(it) - smem) + wg * 1024);
+    const int l = lane_opaque(), dv = wg * VR + l / VCH;
+    const uint32_t cap2 = (uint32_t)p.cap * 2;
+    const uint32_t col = (uint32_t)(((l % VCH) ^ vswz(dv)) << 3) + (uint32_t)(split + NS * it) * KB;
+    const uint32_t voff0 = (uint32_t)dv * cap2 + col * 2;
+    const bool vin = col < (uint32_t)p.cap;
 #pragma unroll
-    for (int j = 0; j < VI; ++j) {
-      const int ins = j * GW + wg;
-      const uint32_t off =
-          vin ? voff0 + (uint32_t)(((int64_t)8 * GW * j * p.cap + (int64_t)kb * KB) * 2) : OOB;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsv, (QA_LDS void*)(sv + ins * 1024), 16, off, 0,
-                                               0, 0);
-    }
+    for (int j = 0; j < VI; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsv, (QA_LDS void*)(sv + j * GW * 1024), 16,
+                                               vin ? voff0 + (uint32_t)(VR * GW * j) * cap2 : OOB, 0, 0, 0);
   };
-  // Loads issued by refill(j), in the VALU phase of step j: K(j + 2) into K
-  // slot j & 1 (S(j) has read it) and V(j + 1) into V slot (j + 1) & 1 (P.V of
-  // step j - 1 has read it).  The MFMA phase of step i needs K(i) and V(i - 1),
-  // issued by refill(i - 1); only refill(i)'s loads may still be in flight.
-  auto refill_count = [&](int j) { return (j + 2 < nst ? KI : 0) + (j + 1 < nst ? VI : 0); };
+  // Loads issued by refill(j), in the VALU phase of step j: K(j + NB) into K
+  // slot j % NB (S(j) has read it) and V(j + NB - 1) (P.V of step j - 1 has
+  // read its slot).  The MFMA phase of step i needs K(i) and V(i - 1), issued
+  // by refill(i - NB): with NB = 2 refill(i - 1)'s loads may still be in
+  // flight, with NB = 1 nothing.
+  auto refill_count = [&](int j) {
+    return NB == 1 ? 0 : (j + 2 < nst ? KI : 0) + (j + 1 < nst ? VI : 0);
+  };
   auto wait_refill = [&](int c) {
     static_assert(KI == VI, "refill counts are 0, VI or KI + VI");
     if (c == LPS)
@@ -292,10 +309,10 @@ __global__ void __launch_bounds__(NS * REP * 2 * 64) attention_kernel(const Attn
   const int64_t qrow = row0 + rg * 32 + fr;
   u32x4 qf[8];
   {
-    const uint16_t* q = p.q + ((int64_t)head * p.rows + qrow) * HD + fh * 8;
+    // (rows past the last repeat it: their outputs are not stored)
+    const uint16_t* q = p.q + ((int64_t)head * p.rows + min(qrow, p.rows - 1)) * HD + fh * 8;
 #pragma unroll
-    for (int s = 0; s < 8; ++s)
-      qf[s] = qrow < p.rows ? *reinterpret_cast<const u32x4*>(q + s * 16) : u32x4{0, 0, 0, 0};
+    for (int s = 0; s < 8; ++s) qf[s] = *reinterpret_cast<const u32x4*>(q + s * 16);
   }
   const int pos = (int)(p.q0 + qrow);                   // this lane's query position
   const int wpos0 = (int)(p.q0 + row0 + rg * 32);       // the wave's first position
@@ -305,8 +322,8 @@ __global__ void __launch_bounds__(NS * REP * 2 * 64) attention_kernel(const Attn
 #pragma unroll
   for (int i = 0; i < 4; ++i) o[i] = f32x16{0};
   float m_run = -INFINITY, l_run = 0.f;
-  f32x16 s[2] = {f32x16{0}, f32x16{0}};
-  u32x4 pf[4], pl[4];
+  f32x16 s[KT] = {};
+  u32x4 pf[2 * KT], pl[2 * KT];
 
   // MFMA phase of step it: P.V of step it - 1 (V slot (it - 1) & 1) and
   // S = K.Q^T of step it (K slot it & 1).  Per 16-deep slice st: the P.V
@@ -316,28 +333,30 @@ __global__ void __launch_bounds__(NS * REP * 2 * 64) attention_kernel(const Attn
   // groups below keep the compiler from sinking the reads next to their use).
   auto mma = [&](auto pv_tag, auto s_tag, int it) {
     constexpr bool PV = decltype(pv_tag)::value, SQ = decltype(s_tag)::value;
-    const unsigned char* sk = kslot(it);
-    const unsigned char* sv = vslot(it - 1);
+    // A fragment row's chunk 2 i + fh sits at ((2 i + fh) ^ swizzle) << 4, so
+    // over i the address is the one of i = 0 with bits 5.. toggled.  The lane's
+    // part is formed here from an opaque copy of the lane index: hoisted out of
+    // the loop, the addresses would spill.
+    const int l = lane_opaque(), r = l & 31, h = l >> 5;
+    const int ka = (int)(kslot(it) - smem) + r * 256 + ((h ^ kswz(r)) << 4);
+    const int va = (int)(vslot(it - 1) - smem) + r * (KB * 2) + ((h ^ vswz(r)) << 4);
     if constexpr (SQ) {
-      s[0] = f32x16{0};
-      s[1] = f32x16{0};
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt) s[kt] = f32x16{0};
     }
     auto rd_v = [&](int st, u32x4* vf) {
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int q = 2 * st + u, dt = q & 3, j = q >> 2;
-        const int d = dt * 32 + fr;
-        vf[u] = *reinterpret_cast<const u32x4*>(sv + d * 128 + (((2 * j + fh) ^ vswz(d)) << 4));
+      for (int u = 0; u < KT; ++u) {
+        const int q = KT * st + u, dt = q & 3, j = q >> 2;
+        vf[u] = *reinterpret_cast<const u32x4*>(smem + (va ^ (j << 5)) + dt * 32 * KB * 2);
       }
     };
     auto rd_k = [&](int st, u32x4* kf) {
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt) {
-        const int r = kt * 32 + fr;
-        kf[kt] = *reinterpret_cast<const u32x4*>(sk + r * 256 + (((2 * st + fh) ^ kswz(r)) << 4));
-      }
+      for (int kt = 0; kt < KT; ++kt)
+        kf[kt] = *reinterpret_cast<const u32x4*>(smem + (ka ^ (st << 5)) + kt * 32 * 256);
     };
-    u32x4 vf[2][2], kf[2][2];
+    u32x4 vf[2][KT], kf[2][KT];
     if constexpr (PV) rd_v(0, vf[0]);
     if constexpr (SQ) rd_k(0, kf[0]);
 #pragma unroll
@@ -349,32 +368,32 @@ __global__ void __launch_bounds__(NS * REP * 2 * 64) attention_kernel(const Attn
       }
       if constexpr (PV) {
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const int q = 2 * st + u, dt = q & 3, j = q >> 2;
+        for (int u = 0; u < KT; ++u) {
+          const int q = KT * st + u, dt = q & 3, j = q >> 2;
           o[dt] = AFmt<DT>::mfma(vf[cur][u], pf[j], o[dt]);
         }
       }
       if constexpr (SQ) {
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt) s[kt] = AFmt<DT>::mfma(kf[cur][kt], qf[st], s[kt]);
+        for (int kt = 0; kt < KT; ++kt) s[kt] = AFmt<DT>::mfma(kf[cur][kt], qf[st], s[kt]);
       }
       if constexpr (PV && PS == 2) {
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const int q = 2 * st + u, dt = q & 3, j = q >> 2;
+        for (int u = 0; u < KT; ++u) {
+          const int q = KT * st + u, dt = q & 3, j = q >> 2;
           o[dt] = AFmt<DT>::mfma(vf[cur][u], pl[j], o[dt]);
         }
       }
     }
     if constexpr (PV && SQ) {
-      // 4 fragment reads, then the slice's 4 or 6 MFMAs, slice by slice
-      __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+      // the fragment reads of a slice, then the MFMAs of the one before
+      __builtin_amdgcn_sched_group_barrier(0x100, 2 * KT, 0);
 #pragma unroll
       for (int st = 0; st < 7; ++st) {
-        __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, PS == 2 ? 6 : 4, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 2 * KT, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, KT * (PS + 1), 0);
       }
-      __builtin_amdgcn_sched_group_barrier(0x008, PS == 2 ? 6 : 4, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, KT * (PS + 1), 0);
     }
   };
 
@@ -384,7 +403,7 @@ __global__ void __launch_bounds__(NS * REP * 2 * 64) attention_kernel(const Attn
     const int kb = split + NS * it;
     if (kb * KB + KB - 1 > wpos0) {  // only blocks that cross this wave's diagonal
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
+      for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
         for (int g = 0; g < 4; ++g)
 #pragma unroll
@@ -395,7 +414,7 @@ __global__ void __launch_bounds__(NS * REP * 2 * 64) attention_kernel(const Attn
     // is applied to the max and, fused, in the exponent: exp2(s sc - m)
     float mx[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
+    for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
       for (int i = 0; i < 16; ++i) mx[i & 3] = fmaxf(mx[i & 3], s[kt][i]);
     const float bm = pair_max(fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3]))) * sc;
@@ -410,7 +429,7 @@ __global__ void __launch_bounds__(NS * REP * 2 * 64) attention_kernel(const Attn
     const float m_b = (m_run == -INFINITY ? 0.f : m_run) - AFmt<DT>::kPBias;
     float rs[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
+    for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         float pv[4];
@@ -432,20 +451,20 @@ __global__ void __launch_bounds__(NS * REP * 2 * 64) attention_kernel(const Attn
     l_run += (rs[0] + rs[1]) + (rs[2] + rs[3]);
   };
 
-  // ---- phases: the two split groups run half a step apart ("ping-pong") ----
-  // A group's step it is an MFMA phase (P.V(it - 1) + S(it)) followed by a
-  // VALU phase (softmax(it)); group 1 runs one phase behind group 0, so on
-  // every SIMD (one wave of each group) one wave's MFMAs overlap the other's
-  // softmax.  Every phase ends in a block barrier, which also orders each
+  // ---- phases: the two halves of the split groups run half a step apart ----
+  // ("ping-pong").  A group's step it is an MFMA phase (P.V(it - 1) + S(it))
+  // followed by a VALU phase (softmax(it)); the upper half of the groups runs
+  // one phase behind the lower, so on every SIMD (one wave of each half) one
+  // wave's MFMAs overlap the other's softmax.  Every phase ends in a block barrier, which also orders each
   // group's LDS reads before the refills that overwrite them.
-  const int n0 = (nkb + 1) / 2, n1 = nkb / 2;
+  const int n0 = (nkb + NS - 1) / NS, n1 = (nkb + NS / 2 - 1) / NS;
   const int phases = max(2 * n0 + 1, 2 * n1 + 2);
   using T_ = std::true_type;
   using F_ = std::false_type;
   if (nst > 0) issue_k(0);  // refill(-2)
-  if (nst > 1) issue_k(1);  // refill(-1): K(1), V(0)
-  if (nst > 0) issue_v(0);
-  if (split == 0) wait_refill(refill_count(-1));
+  if (NB == 2 && nst > 1) issue_k(1);  // refill(-1): K(1), V(0)
+  if (NB == 2 && nst > 0) issue_v(0);
+  if (off == 0) wait_refill(refill_count(-1));
   exec_barrier();
 #ifdef QA_PHASE_STAMPS
   auto stamp = [&](int bucket) {  // charge the cycles since the last mark to a bucket
@@ -458,7 +477,7 @@ __global__ void __launch_bounds__(NS * REP * 2 * 64) attention_kernel(const Attn
   stamp(0);
 #endif
   for (int ph = 0; ph < phases; ++ph) {
-    const int my = ph - split;
+    const int my = ph - off;
 #ifdef QA_PHASE_STAMPS
     int bucket = 3;
 #endif
@@ -476,8 +495,8 @@ __global__ void __launch_bounds__(NS * REP * 2 * 64) attention_kernel(const Attn
         ++nmma;
 #endif
       } else {
-        if (it + 2 < nst) issue_k(it + 2);
-        if (it + 1 < nst) issue_v(it + 1);
+        if (it + NB < nst) issue_k(it + NB);
+        if (it + NB - 1 < nst) issue_v(it + NB - 1);
         softmax(it);
 #ifdef QA_PHASE_STAMPS
         bucket = 2;
@@ -488,7 +507,7 @@ __global__ void __launch_bounds__(NS * REP * 2 * 64) attention_kernel(const Attn
 #ifdef QA_PHASE_STAMPS
     stamp(bucket);
 #endif
-    const int nx = ph + 1 - split;  // this wave's next phase
+    const int nx = ph + 1 - off;  // this wave's next phase
     if (nx >= 0 && (nx & 1) == 0 && (nx >> 1) <= nst) wait_refill(refill_count((nx >> 1) - 1));
     wait_lds();
 #ifdef QA_PHASE_STAMPS
@@ -500,39 +519,70 @@ __global__ void __launch_bounds__(NS * REP * 2 * 64) attention_kernel(const Attn
 #endif
   }
 
-  // ---- merge the two key splits (fixed order) and write the output ----
+  // ---- merge the key splits (in order) and write the output ----
   l_run = pair_sum(l_run);  // both lane halves of the row
   __syncthreads();
-  float* xch = reinterpret_cast<float*>(smem);  // [GW waves][66 values][64 lanes]
-  if (split == 1) {
-    float* dst = xch + (size_t)wg * 66 * 64 + lane;
+  float* xch = reinterpret_cast<float*>(smem);  // [NS - 1][GW waves][66 values][64 lanes]
+  constexpr int XS = GW * 66 * 64;               // one split's floats
+  static_assert((NS - 1) * XS * 4 <= (int)sizeof(smem), "merge buffer");
+  uint16_t* out = p.out + qrow * p.ldo + (int64_t)head * HD;
+  auto store = [&](int dt, int g, const float* v) {
+    const u32x2 pk = {AFmt<DT>::pack2(v[0], v[1]), AFmt<DT>::pack2(v[2], v[3])};
+    *reinterpret_cast<u32x2*>(out + dt * 32 + 8 * g + 4 * fh) = pk;
+  };
+  if (nkb == 1) {  // one key block: split 0 holds every key
+    if (split == 0 && qrow < p.rows) {
+      const float inv = 1.0f / l_run;
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
+      for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) dst[(dt * 16 + v) * 64] = o[dt][v];
-    dst[64 * 64] = m_run;
-    dst[65 * 64] = l_run;
-  }
-  __syncthreads();
-  if (split == 0 && qrow < p.rows) {
-    const float* src = xch + (size_t)wg * 66 * 64 + lane;
-    const float m1 = src[64 * 64], l1 = src[65 * 64];
-    const float mm = fmaxf(m_run, m1);
-    const float mu = mm == -INFINITY ? 0.f : mm;
-    const float a0 = __builtin_amdgcn_exp2f(m_run - mu), a1 = __builtin_amdgcn_exp2f(m1 - mu);
-    const float inv = 1.0f / (l_run * a0 + l1 * a1);
-    uint16_t* out = p.out + qrow * p.ldo + (int64_t)head * HD;
+        for (int g = 0; g < 4; ++g) {
+          float v[4];
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
+          for (int e = 0; e < 4; ++e) v[e] = o[dt][4 * g + e] * inv;
+          store(dt, g, v);
+        }
+    }
+  } else {
+    if (split > 0) {
+      float* dst = xch + (split - 1) * XS + wg * 66 * 64 + lane;
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        float v[4];
+      for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          v[e] = (o[dt][4 * g + e] * a0 + src[(dt * 16 + 4 * g + e) * 64] * a1) * inv;
-        const u32x2 pk = {AFmt<DT>::pack2(v[0], v[1]), AFmt<DT>::pack2(v[2], v[3])};
-        *reinterpret_cast<u32x2*>(out + dt * 32 + 8 * g + 4 * fh) = pk;
+        for (int v = 0; v < 16; ++v) dst[(dt * 16 + v) * 64] = o[dt][v];
+      dst[64 * 64] = m_run;
+      dst[65 * 64] = l_run;
+    }
+    __syncthreads();
+    if (split == 0 && qrow < p.rows) {
+      const float* src = xch + wg * 66 * 64 + lane;
+      float mm = m_run;
+#pragma unroll
+      for (int i = 0; i < NS - 1; ++i) mm = fmaxf(mm, src[i * XS + 64 * 64]);
+      const float mu = mm == -INFINITY ? 0.f : mm;
+      const float a0 = __builtin_amdgcn_exp2f(m_run - mu);
+      float a[NS - 1], sum = l_run * a0;
+#pragma unroll
+      for (int i = 0; i < NS - 1; ++i) {
+        a[i] = __builtin_amdgcn_exp2f(src[i * XS + 64 * 64] - mu);
+        sum += src[i * XS + 65 * 64] * a[i];
       }
+      const float inv = 1.0f / sum;
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          float v[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            v[e] = o[dt][4 * g + e] * a0;
+#pragma unroll
+            for (int i = 0; i < NS - 1; ++i) v[e] += src[i * XS + (dt * 16 + 4 * g + e) * 64] * a[i];
+            v[e] *= inv;
+          }
+          store(dt, g, v);
+        }
+    }
   }
 #ifdef QA_PHASE_STAMPS
   stamp(5);
@@ -548,26 +598,31 @@ __global__ void __launch_bounds__(NS * REP * 2 * 64) attention_kernel(const Attn
 
 }  // namespace
 
-hipError_t launch_attention(int dtype, const AttnParams& p, bool p16, hipStream_t s) {
-  const int rep = p.nqh / p.nkvh;
-  const dim3 grid((unsigned)((p.rows + QT - 1) / QT * p.nkvh));
-  const dim3 block(NS * rep * 2 * 64);
-  void (*k)(AttnParams) = nullptr;
-#define QA_ATTN_PICK(R)                                                                      \
-  if (dtype == QA_BF16)                                                                      \
-    k = p16 ? attention_kernel<QA_BF16, R, 1> : attention_kernel<QA_BF16, R, 2>;             \
-  else                                                                                       \
-    k = p16 ? attention_kernel<QA_F16, R, 1> : attention_kernel<QA_F16, R, 2>;
-  if (rep == 2) {
-    QA_ATTN_PICK(2)
-  } else if (rep == 1) {
-    QA_ATTN_PICK(1)
-  } else {
-    return hipErrorInvalidValue;  // rejected by qa_attention_prefill's validation
-  }
-#undef QA_ATTN_PICK
-  hipLaunchKernelGGL(k, grid, block, 0, s, p);
+namespace {
+
+template <int DT, int REP, int PS, int RG, int NS, int NB>
+hipError_t launch_shape(const AttnParams& p, hipStream_t s) {
+  const dim3 grid((unsigned)((p.rows + 32 * RG - 1) / (32 * RG) * p.nkvh));
+  hipLaunchKernelGGL((attention_kernel<DT, REP, PS, RG, NS, NB>), grid, dim3(NS * REP * RG * 64), 0, s, p);
   return hipGetLastError();
+}
+
+template <int DT, int PS>
+hipError_t launch_ps(const AttnParams& p, hipStream_t s) {
+  const int rep = p.nqh / p.nkvh;
+  if (rep == 1) return launch_shape<DT, 1, PS, 2, 2, 2>(p, s);
+  if (rep != 2) return hipErrorInvalidValue;  // rejected by qa_attention_prefill's validation
+  // 32-row blocks while the 64-row ones would not fill the 256 CUs (the
+  // figures are at the top of the file)
+  if ((p.rows + 63) / 64 * p.nkvh <= 256) return launch_shape<DT, 2, PS, 1, 4, 1>(p, s);
+  return launch_shape<DT, 2, PS, 2, 2, 2>(p, s);
+}
+
+}  // namespace
+
+hipError_t launch_attention(int dtype, const AttnParams& p, bool p16, hipStream_t s) {
+  if (dtype == QA_BF16) return p16 ? launch_ps<QA_BF16, 1>(p, s) : launch_ps<QA_BF16, 2>(p, s);
+  return p16 ? launch_ps<QA_F16, 1>(p, s) : launch_ps<QA_F16, 2>(p, s);
 }
 
 }  // namespace qa

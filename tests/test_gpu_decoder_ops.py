@@ -189,6 +189,26 @@ def test_attention(ctx, pkg, orc, dtype, mode, rows, q0, cap, nqh, nkvh):
 
 
 @DTYPES
+@pytest.mark.parametrize("rows,q0,cap,nqh,nkvh", [
+    (32, 0, 48, 4, 2),        # 32-row blocks: one key block, one split with keys
+    (31, 33, 64, 4, 2),       # ... from a later position
+    (65, 60, 128, 4, 2),      # two key blocks over the four splits
+    (97, 159, 256, 4, 2),     # four: one step each, the last row block one row
+    (33, 288, 336, 4, 2),     # six: two splits take a second step
+    (128, 0, 128, 256, 128),  # 256 blocks of 64 rows: the last 32-row grid
+    (129, 0, 144, 256, 128),  # 384: 64-row blocks, the last one one row
+    (129, 70, 208, 256, 128),
+])
+def test_attention_block_shapes(ctx, pkg, orc, dtype, rows, q0, cap, nqh, nkvh):
+    """Both block shapes at the edges of their row blocks, key blocks and
+    splits, and the two sides of the line between them."""
+    q, kc, vc = _attn_inputs(orc, dtype, rows, q0, cap, nqh, nkvh, rows * 5 + q0)
+    got = _attn_gpu(ctx, pkg, dtype, q, kc, vc, q0, ld_pad=8)
+    want = orc.attention(dtype, q, kc, vc, q0)
+    assert_attention(got, want, q, kc, vc, q0, orc, dtype)
+
+
+@DTYPES
 def test_attention_peaked_scores(ctx, pkg, orc, dtype):
     """Score std ~ 6: the running max moves often and most weights are tiny."""
     rows, q0, cap, nqh, nkvh = 192, 64, 256, 16, 8
