@@ -155,14 +155,27 @@ int validate(const qa_linear_desc* d) {
 // 64-deep k stage of one tile with one block per CU (the L2 -> LDS stream
 // sets it, not the matrix cores), and the fixed cost of a tile (block start
 // skew + prologue fill + epilogue), in microseconds.
-double stage_us(int tile) {
+//
+// The small tiles' stages are cheaper while much of the chip is idle: one CU
+// streams 110-140 GB/s, all 256 together 16-21 TB/s.  Their cost is `idle` up
+// to 45% of the CUs and rises to `full` at 90% (repeated launches, N = 896 and
+// 1024, K = 896 .. 7680, 26 .. 1024 rows; 64 x 64 P2, (time - 3 us) / stages:
+// 0.125-0.14 us up to 112 blocks, 0.14-0.15 at 128, 0.17-0.19 at 182-208,
+// 0.18-0.21 at 224-256).
+double stage_us(int tile, int64_t units, int num_cus) {
+  const double busy = (double)std::min<int64_t>(units, num_cus) / num_cus;
+  auto between = [&](double idle, double full) {
+    return idle + (full - idle) * std::min(1.0, std::max(0.0, (busy - 0.45) / 0.45));
+  };
   switch (tile) {
+    case qa::TILE_64x64: return between(0.155, 0.25);
+    case qa::TILE_64x64_P2: return between(0.135, 0.21);
+    case qa::TILE_32x64_P2: return between(0.115, 0.135);
+    case qa::TILE_32x32_P2: return between(0.09, 0.10);
     case qa::TILE_256x128:
     case qa::TILE_128x256: return 0.95;
     case qa::TILE_128x192: return 0.72;
     case qa::TILE_64x128: return 0.36;
-    case qa::TILE_64x64: return 0.25;
-    case qa::TILE_64x64_P2: return 0.21;
     case qa::TILE_256x256: return 1.75;
     // 256 x 192 (set between its neighbours; picked for the tower's qkv,
     // where it measured 31.0 against 34.9 us on 128 x 192)
@@ -172,13 +185,20 @@ double stage_us(int tile) {
 }
 // 64-deep planes per ring stage: a split's k range runs in whole stages (the
 // planes past its end read zeros), so its cost rounds up to that multiple.
-int planes(int tile) { return tile == qa::TILE_64x64_P2 ? 2 : 1; }
+int planes(int tile) {
+  return tile == qa::TILE_64x64_P2 || tile == qa::TILE_32x64_P2 || tile == qa::TILE_32x32_P2 ? 2 : 1;
+}
 double stages_of(int tile, int64_t kchunk) {
   const int64_t pl = planes(tile);
   return (double)(((kchunk + 63) / 64 + pl - 1) / pl * pl);
 }
-constexpr double kTileFixedUs = 3.0;
-constexpr double kLaunchUs = 2.0;       // one more kernel in the stream (split-K reduce)
+// (the 32-row tiles' fixed cost against 64 x 64 P2's, from the same launches)
+double tile_fixed_us(int tile) {
+  return tile == qa::TILE_32x64_P2 ? 3.2 : tile == qa::TILE_32x32_P2 ? 2.85 : 3.0;
+}
+// One more kernel in the stream (split-K reduce): 3.4-4.8 us at 61-512 rows x
+// 1024 columns, its launch included.
+constexpr double kLaunchUs = 3.5;
 constexpr double kReduceGBs = 3000.0;   // split-K reduce kernel, partials from L2/MALL
 
 // Tile / split-K choice: the modelled time of each candidate is
@@ -205,7 +225,7 @@ qa::Plan plan_linear(const qa_linear_desc& d, int num_cus, size_t max_ws_floats 
   // every tile shape of the plain loader (TILE_256x160 is the conv loader's)
   int cands[] = {qa::TILE_128x128, qa::TILE_256x128, qa::TILE_128x256, qa::TILE_64x128,
                  qa::TILE_64x64,   qa::TILE_128x192, qa::TILE_256x256, qa::TILE_64x64_P2,
-                 qa::TILE_256x192};
+                 qa::TILE_256x192, qa::TILE_32x64_P2, qa::TILE_32x32_P2};
   int ncand = (int)(sizeof cands / sizeof cands[0]);
   if (pl.transb) ncand = 1;  // the conv operand path has one tile shape
   if (forced_tile >= 0 && forced_tile < qa::TILE_COUNT && forced_tile != qa::TILE_256x160 &&
@@ -215,6 +235,10 @@ qa::Plan plan_linear(const qa_linear_desc& d, int num_cus, size_t max_ws_floats 
   }
   double best = 1e300;
   for (int ci = 0; ci < ncand; ++ci) {
+    if (silu && cands[ci] == qa::TILE_32x32_P2) {  // no room for a gate and an up subtile
+      if (ncand == 1) cands[ci] = qa::TILE_32x64_P2;
+      else continue;
+    }
     const qa::TileShape ts = qa::tile_shape(cands[ci]);
     const int64_t tbn = silu ? ts.bn / 2 : ts.bn;
     const int64_t tm = (M + ts.bm - 1) / ts.bm, tn = (nout + tbn - 1) / tbn;
@@ -229,7 +253,8 @@ qa::Plan plan_linear(const qa_linear_desc& d, int num_cus, size_t max_ws_floats 
       if (splits > 1 && forced_splits <= 0 && (size_t)(splits * M * N) > max_ws_floats) break;
       const int64_t units = tiles * splits;
       const int64_t rounds = (units + num_cus - 1) / num_cus;
-      double cost = (double)rounds * (kTileFixedUs + stages_of(cands[ci], kchunk) * stage_us(cands[ci]));
+      double cost = (double)rounds * (tile_fixed_us(cands[ci]) +
+                                      stages_of(cands[ci], kchunk) * stage_us(cands[ci], units, num_cus));
       if (splits > 1)
         cost += kLaunchUs + (double)(splits * 4 + 2) * (double)M * (double)N / (kReduceGBs * 1e3);
       if (cost < best * 0.999) {
@@ -325,7 +350,7 @@ qa::Plan plan_conv(int64_t M, int64_t N, int64_t K, bool gelu, int num_cus) {
     const qa::TileShape ts = qa::tile_shape(tile);
     const int64_t tm = (M + ts.bm - 1) / ts.bm, tn = (N + ts.bn - 1) / ts.bn;
     const int64_t rounds = (tm * tn + num_cus - 1) / num_cus;
-    const double cost = (double)rounds * (kTileFixedUs + (double)pl.kchunk / 64.0 * conv_stage_us(tile));
+    const double cost = (double)rounds * (tile_fixed_us(tile) + (double)pl.kchunk / 64.0 * conv_stage_us(tile));
     if (cost < best * 0.999) {
       best = cost;
       pl.tile = tile;

@@ -420,8 +420,13 @@ __global__ void __launch_bounds__(64 * (WGM * WGN * KG + PW)) gemm_dma_kernel(co
   constexpr int SPG = 4 * PL / KG;           // 16-deep slices per group per stage
   constexpr int WTM = BM / WGM, WTN = BN / WGN;
   constexpr int FM = WTM / 32, FN = WTN / 32;
-  constexpr int AJ = BM / (8 * NW), BJ = BN / (8 * NW);  // DMA instructions per wave per stage
-  constexpr int LPS = (AJ + BJ) * PL;
+  // DMA-issuing waves per plane: all of them fill every plane, or, where a
+  // plane's 8-row groups are too few for that (32-row tiles), NW / PL each
+  // fill a plane of their own.
+  constexpr bool PSPLIT = BM < 8 * NW;
+  constexpr int NWP = PSPLIT ? NW / PL : NW;
+  constexpr int AJ = BM / (8 * NWP), BJ = BN / (8 * NWP);  // DMA instructions per wave per plane
+  constexpr int LPS = (AJ + BJ) * (PSPLIT ? 1 : PL);       // ... per stage
   constexpr int SA = BM * 128, PLANE = (BM + BN) * 128, STAGE = PLANE * PL;
   constexpr int SK = BK * PL;  // k elements per ring stage
   // Epilogue staging: the f32 tile (rows padded by 4 floats) in EP row passes.
@@ -430,7 +435,8 @@ __global__ void __launch_bounds__(64 * (WGM * WGN * KG + PW)) gemm_dma_kernel(co
   constexpr int SMEM = S * STAGE > BM / EP * LDT * 4 ? S * STAGE : BM / EP * LDT * 4;
   static_assert(KG == 1 || KG == 2 || KG == 4, "k groups");
   static_assert(FM >= 1 && FN >= 1 && AJ >= 1 && BJ >= 1, "tile shape");
-  static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "DMA row groups");
+  static_assert(BM % (8 * NWP) == 0 && BN % (8 * NWP) == 0, "DMA row groups");
+  static_assert(!PSPLIT || (NW % PL == 0 && PW > 0), "planes of their own");
   static_assert(EPI != EPI_SILU || BN % 64 == 0, "SiLU tiles hold whole gate / up subtiles");
   static_assert(S >= 2 && (S - 1) * LPS < 64, "pipeline depth");
   static_assert(KG == 1 || (KG - 1) * 4 * BM * BN <= SMEM, "reduction buffer");
@@ -443,7 +449,9 @@ __global__ void __launch_bounds__(64 * (WGM * WGN * KG + PW)) gemm_dma_kernel(co
   const int wave = tid >> 6;
   const bool mma_wave = PW == 0 || wave < NMW;
   const bool dma_wave = PW == 0 || wave >= NMW;
-  const int dwave = PW == 0 ? wave : (wave >= NMW ? wave - NMW : 0);  // index among DMA waves
+  const int dwave_all = PW == 0 ? wave : (wave >= NMW ? wave - NMW : 0);  // index among DMA waves
+  const int dwave = PSPLIT ? dwave_all % NWP : dwave_all;  // ... among its plane's
+  const int dplane = PSPLIT ? dwave_all / NWP : 0;       // its plane (all planes unless PSPLIT)
   const int kg = mma_wave ? wave / GW : KG, w4 = wave % GW;  // producers: no k group
   const int wm = w4 % WGM, wn = w4 / WGM;
   const int fr = lane & 31, fh = lane >> 5;  // fragment row, k-chunk parity
@@ -524,7 +532,7 @@ __global__ void __launch_bounds__(64 * (WGM * WGN * KG + PW)) gemm_dma_kernel(co
   }
 
   // Per-lane byte offsets at k = 0 of the row chunk this lane fetches: lane l
-  // of DMA instruction j fills LDS row r = (NW*j + dwave)*8 + l/8 at physical
+  // of DMA instruction j fills LDS row r = (NWP*j + dwave)*8 + l/8 at physical
   // chunk l%8, so it fetches logical chunk (l%8) ^ swz(r).
   const int lrow = lane >> 3, pchunk = lane & 7;
   uint32_t aoff[AJ], woff[BJ];
@@ -533,7 +541,7 @@ __global__ void __launch_bounds__(64 * (WGM * WGN * KG + PW)) gemm_dma_kernel(co
   int cg[AJ], cic[AJ];             // CV: tap and channel of the lane's chunk in the next plane issued
 #pragma unroll
   for (int j = 0; j < AJ; ++j) {
-    const int r = (j * NW + dwave) * 8 + lrow;
+    const int r = (j * NWP + dwave) * 8 + lrow;
     const int m = m0 + r;
     akc[j] = (pchunk ^ swz(r)) * 8;
     aoff[j] = m < p.M ? (uint32_t)(((int64_t)m * p.lda + akc[j]) * 2) : OOB;
@@ -550,7 +558,7 @@ __global__ void __launch_bounds__(64 * (WGM * WGN * KG + PW)) gemm_dma_kernel(co
   }
 #pragma unroll
   for (int j = 0; j < BJ; ++j) {
-    const int r = (j * NW + dwave) * 8 + lrow;
+    const int r = (j * NWP + dwave) * 8 + lrow;
     const int n = w_row<BN, EPI>(p, tn, r);
     wkc[j] = (pchunk ^ swz(r)) * 8;
     woff[j] = n >= 0 ? (uint32_t)(((int64_t)n * p.ldb + wkc[j]) * 2) : OOB;
@@ -560,11 +568,13 @@ __global__ void __launch_bounds__(64 * (WGM * WGN * KG + PW)) gemm_dma_kernel(co
   // the wave index in a scalar register it is scalar arithmetic, instead of a
   // v_readfirstlane (and its hazard wait) per instruction.
   const int dwave_s = wave_uniform(dwave);
+  const int dplane_s = PSPLIT ? wave_uniform(dplane) : 0;
   // One ring stage's DMA, each chunk checked against the k range (rows past
   // M / N carry OOB, which the buffer unit answers with zeros).
   auto issue_checked = [&](int kidx, int buf) {
 #pragma unroll
-    for (int pl = 0; pl < PL; ++pl) {
+    for (int pi = 0; pi < (PSPLIT ? 1 : PL); ++pi) {
+      const int pl = PSPLIT ? dplane_s : pi;
       const int k0 = kbeg + kidx * SK + pl * BK;
       unsigned char* sb = smem + buf * STAGE + pl * PLANE;
 #pragma unroll
@@ -587,13 +597,13 @@ __global__ void __launch_bounds__(64 * (WGM * WGN * KG + PW)) gemm_dma_kernel(co
           const bool ok = k0 + akc[j] < kend && aoff[j] != OOB;
           off = ok ? aoff[j] + (uint32_t)k0 * 2u : OOB;
         }
-        dma16(rsa, sb + (j * NW + dwave_s) * 1024, off);
+        dma16(rsa, sb + (j * NWP + dwave_s) * 1024, off);
       }
 #pragma unroll
       for (int j = 0; j < BJ; ++j) {
         const bool ok = k0 + wkc[j] < kend && woff[j] != OOB;
         const uint32_t off = ok ? woff[j] + (uint32_t)k0 * 2u : OOB;
-        dma16(rsw, sb + SA + (j * NW + dwave_s) * 1024, off);
+        dma16(rsw, sb + SA + (j * NWP + dwave_s) * 1024, off);
       }
     }
   };
@@ -604,15 +614,16 @@ __global__ void __launch_bounds__(64 * (WGM * WGN * KG + PW)) gemm_dma_kernel(co
   auto issue = [&](int kidx, int buf) {
     if (!CV && kbeg + (kidx + 1) * SK <= kend) {
 #pragma unroll
-      for (int pl = 0; pl < PL; ++pl) {
+      for (int pi = 0; pi < (PSPLIT ? 1 : PL); ++pi) {
+        const int pl = PSPLIT ? dplane_s : pi;
         const uint32_t k2 = (uint32_t)(kbeg + kidx * SK + pl * BK) * 2u;
         unsigned char* sb = smem + buf * STAGE + pl * PLANE;
 #pragma unroll
         for (int j = 0; j < AJ; ++j)
-          dma16(rsa, sb + (j * NW + dwave_s) * 1024, aoff[j] + k2);
+          dma16(rsa, sb + (j * NWP + dwave_s) * 1024, aoff[j] + k2);
 #pragma unroll
         for (int j = 0; j < BJ; ++j)
-          dma16(rsw, sb + SA + (j * NW + dwave_s) * 1024, woff[j] + k2);
+          dma16(rsw, sb + SA + (j * NWP + dwave_s) * 1024, woff[j] + k2);
       }
     } else {
       issue_checked(kidx, buf);
@@ -676,7 +687,10 @@ __global__ void __launch_bounds__(64 * (WGM * WGN * KG + PW)) gemm_dma_kernel(co
   // loads sit in the same in-order vmcnt stream right after stage S-1: the
   // waits for stages 1 .. S-1 leave them outstanding (+PFI), and the kernel
   // prefetches only when every ring stage is issued up front (nk >= S).
-  constexpr int PFI = 2;
+  // Fewer MMA waves take more lines each: when the 176 blocks of a 335-row o
+  // projection on 32 x 64 tiles reached 92% of gate|up's 12.6 MB, gate|up took
+  // 14.6 us in the layer; with all of it, 13.1.
+  constexpr int PFI = NMW <= 2 ? 8 : NMW <= 4 ? 4 : 2;
   static_assert((S - 1) * LPS + PFI < 64, "vmcnt with the prefetch loads");
   const bool pf_on = p.pf_bytes > 0 && z == 0 && mma_wave && (PW > 0 || nk >= S);
   uint32_t pfv[PFI] = {};
@@ -1210,6 +1224,22 @@ hipError_t launch_epi(const Plan& plan, const GemmParams& p, int batch, hipStrea
       // 4352-token prefill -3%, the 300 s forward -2% (same box).
       case TILE_128x192: e = launch_dma<DT, 128, 192, 3, EPI, 1, 4>(plan, p, batch, s, ts); break;
       case TILE_256x256: e = launch_dma<DT, 256, 256, 2, EPI, 1, 0, 0, 4>(plan, p, batch, s, ts); break;
+      // 32-row tiles, for outputs too small for 64 x 64 tiles to fill the
+      // chip: two k groups of one wave each (32 x 64 or 32 x 32; four
+      // groups are level), eight producers, four to a plane.  A launch is then bound by its fixed
+      // ~3.5 us and by what one CU can stream (112-124 GB/s), so smaller
+      // tiles on more CUs win until they need a second round.  Against
+      // 64 x 64 P2 with the K splits and the reduce kernel the planner took
+      // before (f16, N = 1024, repeated): K = 2048 at 61 rows 9.5 -> 6.5 us,
+      // at 256 10.8 -> 6.4, at 323 (32 x 64) 10.8 -> 7.6; K = 3072 at 61 rows
+      // 9.9 -> 7.4, at 323 11.2 -> 9.4.
+      case TILE_32x64_P2:
+        e = launch_dma<DT, 32, 64, 5, EPI, 2, 8, 0, 1, 2, 1>(plan, p, batch, s, ts);
+        break;
+      case TILE_32x32_P2:
+        if constexpr (EPI == EPI_SILU) return hipErrorInvalidValue;  // never planned
+        else e = launch_dma<DT, 32, 32, 6, EPI, 2, 8, 0, 1, 2, 1>(plan, p, batch, s, ts);
+        break;
       // 256 x 192: one round where 128 x 192 needs two (the tower's qkv at M = 3900)
       case TILE_256x192:
         e = launch_dma<DT, 256, 192, 2, EPI, 1, 0, 0, 2, 1, 4>(plan, p, batch, s, ts);

@@ -27,6 +27,8 @@ enum TileCfg : int {
   TILE_64x64_P2 = 7, // 64x64 with two 64-deep planes per ring stage (one barrier per 128 k)
   TILE_256x160 = 8,  // implicit-GEMM conv only: 4 x 1 waves of 64(m) x 160(n)
   TILE_256x192 = 9,  // 4 x 2 waves of 64(m) x 96(n), two stages, MMA waves issue the DMA
+  TILE_32x64_P2 = 10,  // two k groups of one 32 x 64 wave, two planes
+  TILE_32x32_P2 = 11,  // two k groups of one 32 x 32 wave, two planes (no SiLU.up)
   TILE_COUNT
 };
 
@@ -44,6 +46,8 @@ inline TileShape tile_shape(int cfg) {
     case TILE_256x256: return {256, 256};
     case TILE_256x160: return {256, 160};
     case TILE_256x192: return {256, 192};
+    case TILE_32x64_P2: return {32, 64};
+    case TILE_32x32_P2: return {32, 32};
     default: return {128, 128};
   }
 }

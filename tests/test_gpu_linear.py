@@ -214,6 +214,36 @@ def test_forced_tiles_and_splits(ctx, pkg, orc, tile, splits, dtype):
 
 
 @pytest.mark.parametrize("dtype", [0, 1], ids=["f16", "bf16"])
+@pytest.mark.parametrize("tile", [10, 11])
+@pytest.mark.parametrize("splits", [1, 3])
+def test_forced_32_row_tiles(ctx, pkg, orc, tile, splits, dtype):
+    """The 32-row tiles as the others above (11 has no SiLU.up: 10 takes it)."""
+    test_forced_tiles_and_splits(ctx, pkg, orc, tile, splits, dtype)
+
+
+@pytest.mark.parametrize("dtype", [0, 1], ids=["f16", "bf16"])
+@pytest.mark.parametrize("tile", [10, 11])
+@pytest.mark.parametrize("m,n,k", [(1, 4, 8), (31, 36, 72), (33, 60, 120), (32, 64, 128), (65, 100, 1544)])
+def test_32_row_tile_edges(ctx, pkg, orc, tile, m, n, k, dtype):
+    """Rows, columns and k at the edges of the 32-row tiles: k ranges inside
+    one 16-deep slice group, one plane, one stage, and past the ring; residual
+    and bias (the preloaded words) and plain."""
+    rng = np.random.default_rng(m * n + k + tile + dtype)
+    a, w = _case(rng, orc, dtype, m, n, k, w_std=0.1)
+    c0 = _h16(orc, rng.standard_normal((m, n)), dtype)
+    bias = _h16(orc, 0.1 * rng.standard_normal(n), dtype)
+    os.environ["QA_TILE"] = str(tile)
+    try:
+        got = _run(ctx, pkg, dtype, a, w, c0, flags=pkg.ACCUMULATE, bias=bias)
+        plain = _run(ctx, pkg, dtype, a, w, c0)
+    finally:
+        del os.environ["QA_TILE"]
+    exact = orc.linear(dtype, a, w, c0.copy(), flags=orc.ACCUMULATE | orc.EXACT, bias=bias)
+    assert_parity(got, exact, orc, dtype, ulp_tol=1)
+    assert_parity(plain, orc.linear(dtype, a, w, np.zeros_like(c0), flags=orc.EXACT), orc, dtype, ulp_tol=1)
+
+
+@pytest.mark.parametrize("dtype", [0, 1], ids=["f16", "bf16"])
 @pytest.mark.parametrize("group_m", [1, 3, 5, 8, 1000])
 @pytest.mark.parametrize("tile,splits", [(4, 1), (0, 1), (3, 2), (5, 1), (6, 1), (7, 1), (7, 3),
                                          (9, 1), (9, 2)])

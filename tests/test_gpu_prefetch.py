@@ -53,6 +53,13 @@ def test_hint_with_k_shorter_than_the_ring(ctx, pkg, orc, hint_buf, dtype):
     _hint_case(ctx, pkg, orc, hint_buf, 9, 1, 64, dtype)
 
 
+@pytest.mark.parametrize("dtype", [0, 1], ids=["f16", "bf16"])
+@pytest.mark.parametrize("k", [64, 1216])
+@pytest.mark.parametrize("tile,splits", [(10, 1), (11, 1), (10, 3)])
+def test_hint_on_32_row_tiles(ctx, pkg, orc, hint_buf, tile, splits, k, dtype):
+    _hint_case(ctx, pkg, orc, hint_buf, tile, splits, k, dtype)
+
+
 def _hint_case(ctx, pkg, orc, hint_buf, tile, splits, k, dtype):
     rng = np.random.default_rng(7000 + 10 * tile + splits + k + dtype)
     m, n = 300, 512
