@@ -5,21 +5,21 @@
 // bias_gelu, src/audio_encoder_gpu.rs:1165-1201,1714-1794).  With one input
 // channel the im2col row of an output pixel is 9 scattered values, which the
 // implicit GEMM's 16-byte channel chunks cannot fetch.  The 9-tap dot
-// products run on the matrix cores as a K = 16 product (taps 9..15 zero): a
-// wave multiplies 32 output pixels by the weights of 32 output channels per
-// v_mfma_f32_32x32x16, every product of two 16-bit values exact in f32.  What
-// is left on the VALU per output is the bias add, the erf GELU (a reciprocal
-// and an exponential, both at a quarter of the full rate, and ~15 more
-// operations) and the rounding: over the 300-chunk stem (461 M outputs) about
-// 0.3 ms of the 256 CUs' VALU issue at 2.4 GHz, against ~30 slots per
-// output with the taps on the VALU as well (0.43 ms measured before, 0.35
-// after).
+// products run on the matrix cores as a K = 16 product (taps 9..15 zero), with
+// the bias as the accumulator's start: a wave multiplies 32 output pixels by
+// the weights of 32 output channels per v_mfma_f32_32x32x16, every product of
+// two 16-bit values exact in f32.  What is left on the VALU per output is the
+// erf GELU (14 issue slots) and the rounding, and that bounds the kernel: over
+// the 300-chunk stem (461 M outputs) about 0.2 ms of the 256 CUs' VALU issue
+// at 2.2 GHz, more than the 922 MB it writes.
 //
-// A block takes 128 output pixels (32 per wave) x every output channel: the
-// weights sit in LDS as 16 taps per channel (zero-padded), the bias as f32;
+// A block takes 128 output pixels (32 per wave) x a group of channel tiles;
 // each lane holds one pixel's taps as the MFMA's B fragment and, per channel
-// tile, 16 of that pixel's outputs (4 runs of 4 channels), which leave as
-// 8-byte stores.
+// tile, 16 of that pixel's outputs, which leave as two 16-byte stores after a
+// swap between the two halves of the wave.  The weights come straight from
+// global memory in the A fragment's layout (15 KB at 480 channels: a channel's
+// 16 taps are one 32-byte row), one tile ahead; staging them in LDS as 9
+// two-byte loads per channel cost every block ~8 us.
 #include "qa_internal.h"
 
 namespace qa {
@@ -50,16 +50,15 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 template <int DT>
-__device__ __forceinline__ f32x16 mfma(u32x4 a, u32x4 b) {
+__device__ __forceinline__ f32x16 mfma(u32x4 a, u32x4 b, f32x16 c) {
   if constexpr (DT == QA_F16)
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
-                                                  __builtin_bit_cast(f16x8, b), f32x16{0}, 0, 0, 0);
+                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
   else
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
-                                                   __builtin_bit_cast(bf16x8, b), f32x16{0}, 0, 0, 0);
+                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
 // MFMA lane layout (v_mfma_f32_32x32x16, A = 32 channels x 16 taps, B = 16
@@ -67,17 +66,21 @@ __device__ __forceinline__ f32x16 mfma(u32x4 a, u32x4 b) {
 // 8h .. 8h + 7 of channel r (A) and of pixel r (B), and receives pixel r's
 // outputs for channels 8g + 4h + {0..3}, g = 0..3.
 template <int DT, bool GELU>
-__global__ void __launch_bounds__(256) conv1_kernel(const Conv1Params p) {
-  __shared__ __attribute__((aligned(16))) uint16_t ws[kMaxCout * 16];
+__global__ void __launch_bounds__(256) conv1_kernel(const Conv1Params p, int group_tiles) {
   __shared__ __attribute__((aligned(16))) float bs[kMaxCout];
-  const int ntile = (p.c_out + 31) / 32;
-  for (int i = threadIdx.x; i < ntile * 32 * 16; i += 256) {
-    const int c = i >> 4, t = i & 15;
-    ws[i] = c < p.c_out && t < 9 ? p.w[(int64_t)c * p.ldw + t] : (uint16_t)0;
-  }
-  for (int i = threadIdx.x; i < ntile * 32; i += 256)
+  const int ct0 = (int)blockIdx.y * group_tiles;
+  const int ct1 = min((p.c_out + 31) / 32, ct0 + group_tiles);
+  for (int i = ct0 * 32 + threadIdx.x; i < ct1 * 32; i += 256)
     bs[i] = p.bias && i < p.c_out ? widen<DT>(p.bias[i]) : 0.f;
   const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+  // channel ct * 32 + r's taps 8h .. 8h + 7 (only tap 8 of the upper eight;
+  // channels past the last repeat it, their outputs are not stored)
+  auto weights = [&](int ct) {
+    const int c = min(ct * 32 + r, p.c_out - 1);
+    const u32x4 w = *reinterpret_cast<const u32x4*>(p.w + (int64_t)c * p.ldw + 8 * h);
+    return h == 0 ? w : u32x4{w.x & 0xffffu, 0, 0, 0};
+  };
+  u32x4 aop = weights(ct0);
   const int64_t m = (int64_t)blockIdx.x * kPix + (threadIdx.x >> 6) * 32 + r;
   // this lane's taps 8h .. 8h + 7 of pixel m (zeros past tap 8, in the
   // padding and past the last pixel)
@@ -103,40 +106,33 @@ __global__ void __launch_bounds__(256) conv1_kernel(const Conv1Params p) {
   const u32x4 bop = {tv[0], tv[1], tv[2], tv[3]};
   __syncthreads();
   uint16_t* y = p.y + m * p.c_out;
-  // Per channel tile: bias, GELU and the rounding of the lane's 16 outputs,
-  // with no branch between them so their instruction chains interleave.
-  auto tile = [&](int ct, float (&v)[16]) {
-    const u32x4 aop = *reinterpret_cast<const u32x4*>(ws + (ct * 32 + r) * 16 + 8 * h);
-    const f32x16 acc = mfma<DT>(aop, bop);
+  for (int ct = ct0; ct < ct1; ++ct) {
+    f32x16 acc;
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       const f32x4 b4 = *reinterpret_cast<const f32x4*>(bs + ct * 32 + 8 * g + 4 * h);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float a = acc[4 * g + e] + b4[e];
-        v[4 * g + e] = GELU ? gelu_erf(a) : a;
-      }
+      for (int e = 0; e < 4; ++e) acc[4 * g + e] = b4[e];
     }
-  };
-  auto store = [&](int c, const float* v) {
-    *reinterpret_cast<u32x2*>(y + c) = u32x2{pack2<DT>(v[0], v[1]), pack2<DT>(v[2], v[3])};
-  };
-  const int full = p.c_out / 32;  // tiles of 32 channels
-  for (int ct = 0; ct < full; ++ct) {
-    float v[16];
-    tile(ct, v);
-    if (m < p.M) {
+    acc = mfma<DT>(aop, bop, acc);
+    if (ct + 1 < ct1) aop = weights(ct + 1);
+    // GELU and rounding of the lane's 16 outputs, with no branch between them
+    // so their instruction chains interleave
+    uint32_t o[8];
 #pragma unroll
-      for (int g = 0; g < 4; ++g) store(ct * 32 + 8 * g + 4 * h, v + 4 * g);
+    for (int i = 0; i < 8; ++i) {
+      const float a = acc[2 * i], b = acc[2 * i + 1];
+      o[i] = GELU ? pack2<DT>(gelu_erf(a), gelu_erf(b)) : pack2<DT>(a, b);
     }
-  }
-  if (full < ntile) {  // c_out % 32 channels left: runs of 4, all in or all out
-    float v[16];
-    tile(full, v);
+    // runs 2k and 2k + 1 (channels 16 k + 4 h .. and 16 k + 8 + 4 h ..): swapping
+    // the upper half's first run with the lower half's second leaves lane h
+    // with channels 16 k + 8 h .. + 7
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int c = full * 32 + 8 * g + 4 * h;
-      if (m < p.M && c < p.c_out) store(c, v + 4 * g);
+    for (int k = 0; k < 2; ++k) {
+      const auto x = __builtin_amdgcn_permlane32_swap(o[4 * k], o[4 * k + 2], false, false);
+      const auto z = __builtin_amdgcn_permlane32_swap(o[4 * k + 1], o[4 * k + 3], false, false);
+      const int c = ct * 32 + 16 * k + 8 * h;  // c_out % 8 == 0: all in or all out
+      if (m < p.M && c < p.c_out) *reinterpret_cast<u32x4*>(y + c) = u32x4{x[0], z[0], x[1], z[1]};
     }
   }
 }
@@ -146,13 +142,19 @@ __global__ void __launch_bounds__(256) conv1_kernel(const Conv1Params p) {
 hipError_t launch_conv1(int dtype, const Conv1Params& p, hipStream_t s) {
   if (p.c_out > kMaxCout) return hipErrorInvalidValue;  // rejected by validation
   const unsigned blocks = (unsigned)((p.M + kPix - 1) / kPix);
-  const dim3 g(blocks), t(256);
+  // All of a pixel's channels in one block where that gives the chip several
+  // blocks per CU in each of a few rounds; else groups of five tiles (160
+  // channels), so that the last round of a short clip is not mostly idle:
+  // 15 chunks (375 pixel blocks) 33 -> 19.7 us with all of this file's changes;
+  // one group at 300 chunks (7500) 340 -> 273 us.
+  const int tiles = (p.c_out + 31) / 32, group = blocks >= 2048 ? tiles : 5;
+  const dim3 g(blocks, (unsigned)((tiles + group - 1) / group)), t(256);
   if (dtype == QA_BF16) {
-    if (p.gelu) hipLaunchKernelGGL((conv1_kernel<QA_BF16, true>), g, t, 0, s, p);
-    else hipLaunchKernelGGL((conv1_kernel<QA_BF16, false>), g, t, 0, s, p);
+    if (p.gelu) hipLaunchKernelGGL((conv1_kernel<QA_BF16, true>), g, t, 0, s, p, group);
+    else hipLaunchKernelGGL((conv1_kernel<QA_BF16, false>), g, t, 0, s, p, group);
   } else {
-    if (p.gelu) hipLaunchKernelGGL((conv1_kernel<QA_F16, true>), g, t, 0, s, p);
-    else hipLaunchKernelGGL((conv1_kernel<QA_F16, false>), g, t, 0, s, p);
+    if (p.gelu) hipLaunchKernelGGL((conv1_kernel<QA_F16, true>), g, t, 0, s, p, group);
+    else hipLaunchKernelGGL((conv1_kernel<QA_F16, false>), g, t, 0, s, p, group);
   }
   return hipGetLastError();
 }

@@ -75,36 +75,42 @@ __device__ __forceinline__ int fastdiv(int n, FastDiv f) {
   return (int)(((uint64_t)(uint32_t)n * f.m) >> f.p);
 }
 
-// erf-form GELU, 0.5 x (1 + erf(x / sqrt 2)), with erf from Abramowitz &
-// Stegun 7.1.26 (|error| <= 1.5e-7) on v_exp_f32 / v_rcp_f32: the form of the
-// reference's `audio_bias_gelu` (src/shaders.rs:2593-2625); the CPU twin calls
-// libm's erff (src/audio_encoder.rs:196-202).
-//   erf(a) = 1 - P(t) e^{-a^2},  t = 1 / (1 + 0.3275911 a),  a >= 0;
-// for x < 0 the factor 1 + erf(x / sqrt 2) = P(t) e^{-a^2} is formed directly,
-// without cancelling against 1.  Arranged for the VALU (15 instructions, two
-// of them quarter-rate transcendentals, against 17): with q = P(t) e^{-a^2} / 2
-// (the coefficients halved, an exact scaling), gelu(x) = max(x, -0) - |x| q
-// for either sign (x - x q for x >= 0, x q for x < 0: no cancellation on the
-// negative side), one FMA that keeps a zero result's sign and propagates NaN;
-// 1/sqrt 2 folds into the reciprocal's FMA and the exponent's constant.
-// (+inf gives NaN through inf * 0, where 0.5 x (2 - q) gave +inf; an f32 sum
-// of 16-bit products does not reach it.)
+// erf-form GELU, x Phi(x) = max(x, 0) - |x| q with q = Phi(-|x|), the upper
+// tail of the normal distribution (the reference's GPU kernel forms the same
+// with erf from Abramowitz & Stegun 7.1.26, src/shaders.rs:2593-2625; its CPU
+// twin calls libm's erff, src/audio_encoder.rs:196-202).  q = 2^P(|x|) with P a
+// degree-8 polynomial fitted to log2 Phi(-a) on [0, 10] (least squares,
+// reweighted towards the minimax of the error in |x| q, and of q's relative
+// error): 11 VALU instructions, one of them a quarter-rate transcendental, 14
+// issue slots.  With 7.1.26's P(t) e^{-a^2} it was 15 and two, 21 slots, and
+// the GELU bounds the stem's first level (300 chunks: 340 -> 273 us, with the
+// rest of that kernel's changes) and fc1's epilogue (3900 rows bf16: 41.8 ->
+// 39.9 us).  Against the exact GELU in f32 arithmetic: 2.4e-7 absolute on
+// [-5, 5] and 1.6e-8 rms over N(0, 1) (7.1.26: 3.3e-7 and 1.7e-8); relative
+// 1.7e-5 down to x = -3, 2.1e-3 to -5.5, 7e-3 to -10 (5e-5, 2.5e-3, 2e-2);
+// below, the value is under 1e-22.  The sign of a zero result is kept, NaN
+// propagates; +inf gives NaN (inf * 0), which an f32 sum of 16-bit products
+// does not reach.
 __device__ __forceinline__ float gelu_erf(float x) {
-  constexpr float h = 0.5f;
   const float ax = fabsf(x);
-  const float t = __builtin_amdgcn_rcpf(fmaf(ax, 0.3275911f * 0.70710678118654752f, 1.0f));
-  const float e = __builtin_amdgcn_exp2f(x * x * (-0.5f * 1.44269504088896341f));  // e^{-a^2}
-  const float p = (((h * 1.061405429f * t - h * 1.453152027f) * t + h * 1.421413741f) * t -
-                   h * 0.284496736f) * t + h * 0.254829592f;
+  float p = fmaf(ax, -6.02775501e-08f, 1.88221534e-07f);
+  p = fmaf(p, ax, 3.7997328e-05f);
+  p = fmaf(p, ax, -0.000805318821f);
+  p = fmaf(p, ax, 0.00817962456f);
+  p = fmaf(p, ax, -0.0535414778f);
+  p = fmaf(p, ax, -0.458688706f);
+  p = fmaf(p, ax, -1.15122461f);
+  const float q = __builtin_amdgcn_exp2f(fmaf(p, ax, -0.999991059f));
   // max(x, -0) as one v_max_f32: fmaxf adds a canonicalising v_max first,
   // which only matters for a NaN x, and a NaN x makes the FMA NaN anyway.
-  // The instruction does not read %2 (e): that operand only orders the
-  // statement after x * x, a compiler instruction reading x, ahead of which
-  // the compiler puts any wait state x's producer needs (an MFMA's result,
-  // in the register-staged GEMM); it puts none ahead of an asm statement.
+  // The instruction does not read %2 (p): that operand only orders the
+  // statement after the first FMA, a compiler instruction reading x, ahead of
+  // which the compiler puts any wait state x's producer needs (an MFMA's
+  // result, in the register-staged GEMM); it puts none ahead of an asm
+  // statement.
   float mx;
-  asm("v_max_f32_e64 %0, %1, neg(0)" : "=v"(mx) : "v"(x), "v"(e));
-  return fmaf(-ax, p * t * e, mx);
+  asm("v_max_f32_e64 %0, %1, neg(0)" : "=v"(mx) : "v"(x), "v"(p));
+  return fmaf(-ax, q, mx);
 }
 
 // x + the f16 value in the low (hi = false) or high half of w, in f32 with
