@@ -305,8 +305,14 @@ void choose_group_m(qa::Plan& pl, int64_t span) {
   }
 }
 
-// The implicit-GEMM convolution: M = output pixels, N = c_out, K = 9 c_in,
-// never split (K is long), on the tile shapes the CV loader is built for.
+// The implicit-GEMM convolution: M = output pixels, N = c_out, K = 9 c_in, on
+// the tile shapes the CV loader is built for.  K is long (4320 at 480
+// channels, 68 stages), so a short clip's few tiles would run its whole loop
+// on part of the chip: there it is split, up to six ways, for f32 partials
+// and the reduce kernel.  Second / third level, f16, unsplit -> split: 2
+// chunks (13 / 4 x 128 rows) 43 -> 20.0 and 35 -> 16.1 us; 5 chunks 36 ->
+// 30.6 and 34 -> 17.2; 15 chunks (third level) 32.7 -> 28.2.  From 25 chunks
+// on the plans are unsplit.
 // The A operand is an input slab that nine taps re-read; at the stem's sizes
 // (a 921 MB input for the second level over 300 chunks) an XCD's range of
 // tiles touches far more of it than its 4 MB L2 holds, so only the tiles
@@ -335,29 +341,40 @@ double conv_stage_us(int tile) {
     default: return 0.74;  // 128 x 128
   }
 }
-qa::Plan plan_conv(int64_t M, int64_t N, int64_t K, bool gelu, int num_cus) {
+qa::Plan plan_conv(int64_t M, int64_t N, int64_t K, bool gelu, int num_cus, size_t max_ws_floats) {
   qa::Plan pl{};
   pl.epi = gelu ? qa::EPI_GELU : qa::EPI_PLAIN;
   pl.conv = true;
   pl.splits = 1;
   pl.kchunk = (int)((K + 63) / 64 * 64);
   double best = 1e300;
-  int forced_tile = -1;
+  int forced_tile = -1, forced_splits = 0;
   if (const char* e = getenv("QA_TILE")) forced_tile = atoi(e);
+  if (const char* e = getenv("QA_SPLITS")) forced_splits = atoi(e);
   for (const int tile : {qa::TILE_128x256, qa::TILE_256x128, qa::TILE_128x128, qa::TILE_256x256,
                          qa::TILE_256x160}) {
     if (forced_tile >= 0 && forced_tile != tile) continue;
     const qa::TileShape ts = qa::tile_shape(tile);
     const int64_t tm = (M + ts.bm - 1) / ts.bm, tn = (N + ts.bn - 1) / ts.bn;
-    const int64_t rounds = (tm * tn + num_cus - 1) / num_cus;
-    const double cost = (double)rounds * (tile_fixed_us(tile) + (double)pl.kchunk / 64.0 * conv_stage_us(tile));
-    if (cost < best * 0.999) {
-      best = cost;
-      pl.tile = tile;
-      pl.tiles_m = (int)tm;
-      pl.tiles_n = (int)tn;
+    for (int64_t want = forced_splits > 0 ? forced_splits : 1; want <= (forced_splits > 0 ? forced_splits : 6);
+         ++want) {
+      const int64_t kchunk = ((K + want - 1) / want + 63) / 64 * 64, splits = (K + kchunk - 1) / kchunk;
+      if (splits > 1 && ((size_t)(splits * M * N) > max_ws_floats || (kchunk < 256 && forced_splits <= 0))) break;
+      const int64_t rounds = (tm * tn * splits + num_cus - 1) / num_cus;
+      double cost = (double)rounds * (tile_fixed_us(tile) + (double)kchunk / 64.0 * conv_stage_us(tile));
+      if (splits > 1)
+        cost += kLaunchUs + (double)(splits * 4 + 2) * (double)M * (double)N / (kReduceGBs * 1e3);
+      if (cost < best * 0.999) {
+        best = cost;
+        pl.tile = tile;
+        pl.tiles_m = (int)tm;
+        pl.tiles_n = (int)tn;
+        pl.splits = (int)splits;
+        pl.kchunk = (int)kchunk;
+      }
     }
   }
+  if (pl.splits > 1) pl.ws_floats = (size_t)pl.splits * (size_t)M * (size_t)N;
   if (best == 1e300) {  // a forced tile the conv path does not have
     pl.tile = qa::TILE_128x128;
     pl.tiles_m = (int)((M + 127) / 128);
@@ -367,10 +384,14 @@ qa::Plan plan_conv(int64_t M, int64_t N, int64_t K, bool gelu, int num_cus) {
   return pl;
 }
 
+bool capturing(qa_ctx* ctx) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(ctx->stream, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
+}
+
 int ensure_workspace(qa_ctx* ctx, size_t floats) {
   if (floats <= ctx->ws_floats) return ok();
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(ctx->stream, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone)
+  if (capturing(ctx))
     return fail(QA_EINVAL,
                 "the context workspace must grow (%zu floats) but the stream is being "
                 "captured; run the same call once before capture",
@@ -852,8 +873,13 @@ int qa_conv2d_3x3s2(qa_ctx* ctx, const qa_conv_desc* d) {
     const hipError_t e = qa::launch_conv1((int)d->dtype, p, ctx->stream);
     return e == hipSuccess ? ok() : hip_fail(e, "qa_conv2d_3x3s2 launch");
   }
-  const qa::Plan plan = plan_conv(M, d->c_out, K, gelu, ctx->num_cus);
+  // A captured call is never split: its replays would go on using a workspace
+  // that a later, larger call replaces, where the unsplit form uses none.
+  qa::Plan plan = plan_conv(M, d->c_out, K, gelu, ctx->num_cus, capturing(ctx) ? 0 : SIZE_MAX);
+  if (plan.splits > 1 && ensure_workspace(ctx, plan.ws_floats))  // no memory for it: run unsplit
+    plan = plan_conv(M, d->c_out, K, gelu, ctx->num_cus, 0);
   qa::GemmParams p{};
+  p.ws = ctx->ws;
   p.a = (const uint16_t*)d->x;
   p.w = (const uint16_t*)d->weight;
   p.c = (uint16_t*)d->y;
@@ -868,7 +894,7 @@ int qa_conv2d_3x3s2(qa_ctx* ctx, const qa_conv_desc* d) {
   p.ldc = (int)d->c_out;
   p.tiles_m = plan.tiles_m;
   p.tiles_n = plan.tiles_n;
-  p.splits = 1;
+  p.splits = plan.splits;
   p.kchunk = plan.kchunk;
   p.group_m = plan.group_m;
   p.cv_c = (int)d->c_in;

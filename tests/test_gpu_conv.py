@@ -93,6 +93,50 @@ def test_conv_tiles_and_no_activation(ctx, pkg, orc, monkeypatch, tile):
     assert_parity(got, want, orc, F16, ulp_tol=1)
 
 
+@pytest.mark.parametrize("dtype", [F16, BF16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("tile,splits", [("0", "2"), ("1", "3"), ("2", "5"), ("6", "2"), ("8", "9"), ("", "")])
+@pytest.mark.parametrize("tmajor", [False, True], ids=["rows_hw", "rows_wh"])
+def test_conv_split_k(ctx, pkg, orc, monkeypatch, dtype, tile, splits, tmajor):
+    """K split over f32 partials and the reduce kernel, on every tile shape
+    (taps and channels of a split start inside a tap; 14 stages, uneven splits),
+    and the planner's own choice at this size: bias, GELU, both row orders."""
+    if tile:
+        monkeypatch.setenv("QA_TILE", tile)
+        monkeypatch.setenv("QA_SPLITS", splits)
+    x, wt, bias = _case(orc, dtype, 2, 20, 18, 96, 200, 7)
+    flags = pkg.QA_CONV_GELU | (pkg.QA_CONV_TOKEN_MAJOR if tmajor else 0)
+    got = _conv_gpu(ctx, pkg, dtype, x, wt, bias, 200, flags)
+    want = orc.conv3x3s2(dtype, x, wt, bias, gelu=True, token_major=tmajor)
+    assert_parity(got, want, orc, dtype, ulp_tol=1)
+    assert np.array_equal(got, _conv_gpu(ctx, pkg, dtype, x, wt, bias, 200, flags))
+
+
+def test_conv_captured_without_workspace(pkg, orc):
+    """On a fresh context a captured convolution runs unsplit (no workspace):
+    every replay within one ulp, also after eager calls grew the workspace."""
+    from hipgraph import Capture
+    x, wt, bias = _case(orc, F16, 2, 20, 18, 96, 200, 7)
+    want = orc.conv3x3s2(F16, x, wt, bias, gelu=True)
+    with pkg.Context(0) as ctx:
+        dx, dw, db = ctx.to_device(x), ctx.to_device(wt), ctx.to_device(bias)
+        dy, dz = ctx.alloc(want.size * 2), ctx.alloc(want.size * 2)
+
+        def run(y):
+            ctx.conv2d_3x3s2(pkg.ConvDesc(dtype=F16, flags=pkg.QA_CONV_GELU, batch=2, h=20, w=18, c_in=96, c_out=200,
+                                          x=int(dx), weight=int(dw), bias=int(db), y=int(y)))
+
+        with Capture(ctx.stream) as cap:
+            run(dy)
+        for _ in range(3):
+            ctx.upload(dy, np.zeros(want.shape, np.uint16))
+            cap.replay()
+            assert_parity(ctx.download(dy, want.shape), want, orc, F16, ulp_tol=1)
+            run(dz)  # eager, split
+            ctx.sync()
+        assert_parity(ctx.download(dz, want.shape), want, orc, F16, ulp_tol=1)
+        cap.close()
+
+
 def test_conv_stem_at_300_s(ctx, pkg, orc):
     """conv2 over the 300 chunks of 300 s of audio (240 000 output pixels,
     995 GFLOP): the oracle checks the first, a middle and the last block of 64
