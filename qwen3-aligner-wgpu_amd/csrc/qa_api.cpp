@@ -27,6 +27,11 @@ struct qa_ctx {
   int num_cus = 256;
   float* ws = nullptr;  // split-K partials
   size_t ws_floats = 0;
+  // Split convolutions' partials.  Not in `ws`: that one's address is kept by
+  // captured launches, and a convolution, which needs none for itself, must
+  // not be what replaces it under them.  No captured launch keeps this one's.
+  float* conv_ws = nullptr;
+  size_t conv_ws_floats = 0;
   float* scratch = nullptr;  // this device's copy of `scratch` (qa_linear_noalloc)
   // qa_prefetch_hint: bytes the projection after the next one reads; the next
   // projection launch takes it over and clears it
@@ -407,6 +412,30 @@ int ensure_workspace(qa_ctx* ctx, size_t floats) {
   return ok();
 }
 
+// The split convolutions' partials; false if there is no memory for them (the
+// caller then runs unsplit).  The thread's capture mode is relaxed meanwhile:
+// a convolution on this stream may run while another stream is captured, and
+// an allocation would break that capture.
+bool ensure_conv_workspace(qa_ctx* ctx, size_t floats) {
+  if (floats <= ctx->conv_ws_floats) return true;
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return false;
+  bool have = hipStreamSynchronize(ctx->stream) == hipSuccess;
+  if (have) {
+    if (ctx->conv_ws) (void)hipFree(ctx->conv_ws);
+    ctx->conv_ws = nullptr;
+    ctx->conv_ws_floats = 0;
+    have = hipMalloc(&ctx->conv_ws, floats * sizeof(float)) == hipSuccess;
+    if (have) ctx->conv_ws_floats = floats;
+    else {
+      ctx->conv_ws = nullptr;
+      (void)hipGetLastError();
+    }
+  }
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  return have;
+}
+
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 float* g_scratch[kMaxDevices] = {};
@@ -546,6 +575,7 @@ int qa_ctx_destroy(qa_ctx* ctx) {
   (void)hipSetDevice(ctx->device);
   (void)hipStreamSynchronize(ctx->stream);
   if (ctx->ws) (void)hipFree(ctx->ws);
+  if (ctx->conv_ws) (void)hipFree(ctx->conv_ws);
   const hipError_t e = hipStreamDestroy(ctx->stream);
   delete ctx;
   return e == hipSuccess ? ok() : hip_fail(e, "hipStreamDestroy");
@@ -873,13 +903,13 @@ int qa_conv2d_3x3s2(qa_ctx* ctx, const qa_conv_desc* d) {
     const hipError_t e = qa::launch_conv1((int)d->dtype, p, ctx->stream);
     return e == hipSuccess ? ok() : hip_fail(e, "qa_conv2d_3x3s2 launch");
   }
-  // A captured call is never split: its replays would go on using a workspace
-  // that a later, larger call replaces, where the unsplit form uses none.
+  // A captured call is never split: its replays would go on using partials'
+  // memory that a later, larger call replaces, where the unsplit form uses none.
   qa::Plan plan = plan_conv(M, d->c_out, K, gelu, ctx->num_cus, capturing(ctx) ? 0 : SIZE_MAX);
-  if (plan.splits > 1 && ensure_workspace(ctx, plan.ws_floats))  // no memory for it: run unsplit
+  if (plan.splits > 1 && !ensure_conv_workspace(ctx, plan.ws_floats))
     plan = plan_conv(M, d->c_out, K, gelu, ctx->num_cus, 0);
   qa::GemmParams p{};
-  p.ws = ctx->ws;
+  p.ws = ctx->conv_ws;
   p.a = (const uint16_t*)d->x;
   p.w = (const uint16_t*)d->weight;
   p.c = (uint16_t*)d->y;

@@ -137,6 +137,39 @@ def test_conv_captured_without_workspace(pkg, orc):
         cap.close()
 
 
+def test_conv_leaves_captured_workspace(pkg, orc, monkeypatch):
+    """A split convolution keeps its partials apart from the workspace that a
+    captured split linear uses: the replays stay right after eager convolutions
+    whose partials are larger."""
+    from hipgraph import Capture
+    rng = np.random.default_rng(11)
+    m, n, k = 64, 128, 1024
+    a = _h16(orc, rng.standard_normal((m, k)), F16)
+    w = _h16(orc, rng.standard_normal((n, k)) * 0.05, F16)
+    x, wt, bias = _case(orc, F16, 2, 20, 18, 96, 200, 7)
+    conv_want = orc.conv3x3s2(F16, x, wt, bias, gelu=True)
+    with pkg.Context(0) as ctx:
+        da, dw, dc = ctx.to_device(a), ctx.to_device(w), ctx.alloc(m * n * 2)
+        dx, dk, db, dy = ctx.to_device(x), ctx.to_device(wt), ctx.to_device(bias), ctx.alloc(conv_want.size * 2)
+        lin = pkg.linear_desc(F16, m, n, k, da, dw, dc)
+        conv = pkg.ConvDesc(dtype=F16, flags=pkg.QA_CONV_GELU, batch=2, h=20, w=18, c_in=96, c_out=200,
+                            x=int(dx), weight=int(dk), bias=int(db), y=int(dy))
+        monkeypatch.setenv("QA_SPLITS", "2")
+        ctx.linear(lin)  # grows the workspace
+        want = ctx.download(dc, (m, n))
+        with Capture(ctx.stream) as cap:
+            ctx.linear(lin)
+        for splits in ("2", "5", "3"):
+            monkeypatch.setenv("QA_SPLITS", splits)
+            ctx.conv2d_3x3s2(conv)
+            ctx.upload(dc, np.zeros((m, n), np.uint16))
+            cap.replay()
+            assert np.array_equal(ctx.download(dc, (m, n)), want)
+            ctx.conv2d_3x3s2(conv)  # and the replay leaves the partials alone
+            assert_parity(ctx.download(dy, conv_want.shape), conv_want, orc, F16, ulp_tol=1)
+        cap.close()
+
+
 def test_conv_stem_at_300_s(ctx, pkg, orc):
     """conv2 over the 300 chunks of 300 s of audio (240 000 output pixels,
     995 GFLOP): the oracle checks the first, a middle and the last block of 64
