@@ -25,6 +25,11 @@
 //    10.5, 1024 rows 25.2 -> 17.8, 2048 rows (256 blocks of 64) 42.6 -> 36.1,
 //    2200 rows (280) 46.0 -> 48.3; 771 rows from position 1536 with 16-bit
 //    probabilities 38.8 -> 24.6.  Hence the line at 256 blocks of 64 rows.
+//    Behind a long past the blocks are all about equally long, and 257 to 512
+//    of 32 rows take two full rounds: 8 kv heads, 1200 rows from position
+//    1000 43.0 -> 40.3 us, 1500 51.1 -> 50.6, 2000 58.8 -> 60.9, 4000 91 ->
+//    100, 8000 154 -> 182; 2048 rows from 2000 88 -> 84, 4000 133 -> 133, 8000
+//    223 -> 229.  Hence the 64-row shape there from 1.5 times the rows on.
 //
 // Per key block, per wave (32 query rows):
 //  * S = K . Q^T on v_mfma_f32_32x32x16 (A = 32 keys x 16 d from LDS, B = the
@@ -612,9 +617,12 @@ hipError_t launch_ps(const AttnParams& p, hipStream_t s) {
   const int rep = p.nqh / p.nkvh;
   if (rep == 1) return launch_shape<DT, 1, PS, 2, 2, 2>(p, s);
   if (rep != 2) return hipErrorInvalidValue;  // rejected by qa_attention_prefill's validation
-  // 32-row blocks while the 64-row ones would not fill the 256 CUs (the
+  // 32-row blocks while the 64-row ones would not fill the 256 CUs, unless
+  // they need a second round of blocks about as long as the first (the
   // figures are at the top of the file)
-  if ((p.rows + 63) / 64 * p.nkvh <= 256) return launch_shape<DT, 2, PS, 1, 4, 1>(p, s);
+  const bool one_round = (p.rows + 31) / 32 * p.nkvh <= 256;
+  if (one_round || ((p.rows + 63) / 64 * p.nkvh <= 256 && 2 * p.q0 < 3 * p.rows))
+    return launch_shape<DT, 2, PS, 1, 4, 1>(p, s);
   return launch_shape<DT, 2, PS, 2, 2, 2>(p, s);
 }
 

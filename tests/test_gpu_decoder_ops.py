@@ -198,6 +198,8 @@ def test_attention(ctx, pkg, orc, dtype, mode, rows, q0, cap, nqh, nkvh):
     (128, 0, 128, 256, 128),  # 256 blocks of 64 rows: the last 32-row grid
     (129, 0, 144, 256, 128),  # 384: 64-row blocks, the last one one row
     (129, 70, 208, 256, 128),
+    (65, 97, 176, 256, 128),  # 384 blocks of 32 rows, the past just under 1.5 times the rows
+    (65, 98, 176, 256, 128),  # ... and just over: 64-row blocks
 ])
 def test_attention_block_shapes(ctx, pkg, orc, dtype, rows, q0, cap, nqh, nkvh):
     """Both block shapes at the edges of their row blocks, key blocks and
