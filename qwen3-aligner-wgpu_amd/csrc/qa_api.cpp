@@ -316,8 +316,12 @@ void choose_group_m(qa::Plan& pl, int64_t span) {
 // on part of the chip: there it is split, up to six ways, for f32 partials
 // and the reduce kernel.  Second / third level, f16, unsplit -> split: 2
 // chunks (13 / 4 x 128 rows) 43 -> 20.0 and 35 -> 16.1 us; 5 chunks 36 ->
-// 30.6 and 34 -> 17.2; 15 chunks (third level) 32.7 -> 28.2.  From 25 chunks
-// on the plans are unsplit.
+// 30.6 and 34 -> 17.2; 15 chunks (third level) 32.7 -> 28.2.  Unsplit tiles
+// that leave CUs idle run faster than the model says, so a split has to be
+// modelled under 0.7 of the unsplit plan: with any modelled gain taken, the
+// whole stem over 20 chunks (0.74) took 135.5 us against 134.4 unsplit, 24
+// (0.80) 155.1 against 152.7, 34 (0.98) 220.7 against 212.5; 19 chunks (0.68)
+// 127.5 against 130.5.
 // The A operand is an input slab that nine taps re-read; at the stem's sizes
 // (a 921 MB input for the second level over 300 chunks) an XCD's range of
 // tiles touches far more of it than its 4 MB L2 holds, so only the tiles
@@ -352,7 +356,7 @@ qa::Plan plan_conv(int64_t M, int64_t N, int64_t K, bool gelu, int num_cus, size
   pl.conv = true;
   pl.splits = 1;
   pl.kchunk = (int)((K + 63) / 64 * 64);
-  double best = 1e300;
+  double best = 1e300, unsplit = 1e300;
   int forced_tile = -1, forced_splits = 0;
   if (const char* e = getenv("QA_TILE")) forced_tile = atoi(e);
   if (const char* e = getenv("QA_SPLITS")) forced_splits = atoi(e);
@@ -369,6 +373,8 @@ qa::Plan plan_conv(int64_t M, int64_t N, int64_t K, bool gelu, int num_cus, size
       double cost = (double)rounds * (tile_fixed_us(tile) + (double)kchunk / 64.0 * conv_stage_us(tile));
       if (splits > 1)
         cost += kLaunchUs + (double)(splits * 4 + 2) * (double)M * (double)N / (kReduceGBs * 1e3);
+      else
+        unsplit = std::min(unsplit, cost);
       if (cost < best * 0.999) {
         best = cost;
         pl.tile = tile;
@@ -379,6 +385,8 @@ qa::Plan plan_conv(int64_t M, int64_t N, int64_t K, bool gelu, int num_cus, size
       }
     }
   }
+  if (pl.splits > 1 && forced_splits <= 0 && best > 0.7 * unsplit)
+    return plan_conv(M, N, K, gelu, num_cus, 0);
   if (pl.splits > 1) pl.ws_floats = (size_t)pl.splits * (size_t)M * (size_t)N;
   if (best == 1e300) {  // a forced tile the conv path does not have
     pl.tile = qa::TILE_128x128;
