@@ -312,14 +312,18 @@ __global__ void __launch_bounds__(NS * REP * RG * 64) attention_kernel(const Att
 
   // ---- this wave's 32 query rows, as MFMA B fragments (8 slices of 16 d) ----
   const int64_t qrow = row0 + rg * 32 + fr;
+  // Lanes past the last row repeat it, position and all, and store nothing.  A
+  // position of their own would let them see cache entries that this call
+  // never wrote, and a large score there moves the running max of the
+  // wave's valid rows too (the ballot in softmax).
+  const int64_t lrow = min(qrow, p.rows - 1);
   u32x4 qf[8];
   {
-    // (rows past the last repeat it: their outputs are not stored)
-    const uint16_t* q = p.q + ((int64_t)head * p.rows + min(qrow, p.rows - 1)) * HD + fh * 8;
+    const uint16_t* q = p.q + ((int64_t)head * p.rows + lrow) * HD + fh * 8;
 #pragma unroll
     for (int s = 0; s < 8; ++s) qf[s] = *reinterpret_cast<const u32x4*>(q + s * 16);
   }
-  const int pos = (int)(p.q0 + qrow);                   // this lane's query position
+  const int pos = (int)(p.q0 + lrow);                   // this lane's query position
   const int wpos0 = (int)(p.q0 + row0 + rg * 32);       // the wave's first position
   const float sc = p.scale * kLog2e;
 

@@ -211,6 +211,32 @@ def test_attention_block_shapes(ctx, pkg, orc, dtype, rows, q0, cap, nqh, nkvh):
 
 
 @DTYPES
+@pytest.mark.parametrize("mode", ["split", "p16"])
+@pytest.mark.parametrize("rows,q0,cap,nqh,nkvh", [
+    (33, 240, 320, 16, 8),    # 32-row blocks, four splits: block 4 (keys 256..) is split 0's second
+    (65, 290, 384, 4, 4),     # 64-row blocks, two splits: block 5 is split 1's third
+    (129, 160, 320, 256, 128),  # ... with two q heads
+])
+def test_attention_ignores_stale_cache(ctx, pkg, orc, dtype, mode, rows, q0, cap, nqh, nkvh):
+    """The result does not depend on what an earlier, longer prefill left in
+    the cache past q0 + rows: equal bits over zeros there and over keys that
+    follow the last row's query (scores of several hundred, which would move
+    the running max of any lane that saw them, and with it the rounding of its
+    wave's other rows)."""
+    q, kc, vc = _attn_inputs(orc, dtype, rows, q0, cap, nqh, nkvh, rows * 3 + q0)
+    kend = q0 + rows
+    cols = orc.vperm(cap)[kend:]
+    flags = pkg.QA_ATTN_P16 if mode == "p16" else 0
+    kc[:, kend:] = 0
+    vc[:, :, cols] = 0
+    clean = _attn_gpu(ctx, pkg, dtype, q, kc, vc, q0, flags=flags)
+    last = orc.h16_to_f32(q[::nqh // nkvh, -1], dtype)  # a q head of each kv head
+    kc[:, kend:] = _h16(orc, 50.0 * last, dtype)[:, None]
+    vc[:, :, cols] = _h16(orc, np.full((nkvh, 128, cap - kend), 300.0), dtype)
+    assert np.array_equal(_attn_gpu(ctx, pkg, dtype, q, kc, vc, q0, flags=flags), clean)
+
+
+@DTYPES
 def test_attention_peaked_scores(ctx, pkg, orc, dtype):
     """Score std ~ 6: the running max moves often and most weights are tiny."""
     rows, q0, cap, nqh, nkvh = 192, 64, 256, 16, 8
