@@ -9,7 +9,7 @@
 // the bias as the accumulator's start: a wave multiplies 32 output pixels by
 // the weights of 32 output channels per v_mfma_f32_32x32x16, every product of
 // two 16-bit values exact in f32.  What is left on the VALU per output is the
-// erf GELU (14 issue slots) and the rounding, and that bounds the kernel: over
+// erf GELU (16 issue slots) and the rounding, and that bounds the kernel: over
 // the 300-chunk stem (461 M outputs) about 0.2 ms of the 256 CUs' VALU issue
 // at 2.2 GHz, more than the 922 MB it writes.
 //
@@ -145,8 +145,8 @@ hipError_t launch_conv1(int dtype, const Conv1Params& p, hipStream_t s) {
   // All of a pixel's channels in one block where that gives the chip several
   // blocks per CU in each of a few rounds; else groups of five tiles (160
   // channels), so that the last round of a short clip is not mostly idle:
-  // 15 chunks (375 pixel blocks) 33 -> 19.7 us with all of this file's changes;
-  // one group at 300 chunks (7500) 340 -> 273 us.
+  // 15 chunks (375 pixel blocks) 30.9 -> 19.1 us with all of this file's changes;
+  // one group at 300 chunks (7500) 357 -> 308 us.
   const int tiles = (p.c_out + 31) / 32, group = blocks >= 2048 ? tiles : 5;
   const dim3 g(blocks, (unsigned)((tiles + group - 1) / group)), t(256);
   if (dtype == QA_BF16) {

@@ -79,28 +79,36 @@ __device__ __forceinline__ int fastdiv(int n, FastDiv f) {
 // tail of the normal distribution (the reference's GPU kernel forms the same
 // with erf from Abramowitz & Stegun 7.1.26, src/shaders.rs:2593-2625; its CPU
 // twin calls libm's erff, src/audio_encoder.rs:196-202).  q = 2^P(|x|) with P a
-// degree-8 polynomial fitted to log2 Phi(-a) on [0, 10] (least squares,
-// reweighted towards the minimax of the error in |x| q, and of q's relative
-// error): 11 VALU instructions, one of them a quarter-rate transcendental, 14
-// issue slots.  With 7.1.26's P(t) e^{-a^2} it was 15 and two, 21 slots, and
-// the GELU bounds the stem's first level (300 chunks: 340 -> 273 us, with the
-// rest of that kernel's changes) and fc1's epilogue (3900 rows bf16: 41.8 ->
-// 39.9 us).  Against the exact GELU in f32 arithmetic: 2.4e-7 absolute on
-// [-5, 5] and 1.6e-8 rms over N(0, 1) (7.1.26: 3.3e-7 and 1.7e-8); relative
-// 1.7e-5 down to x = -3, 2.1e-3 to -5.5, 7e-3 to -10 (5e-5, 2.5e-3, 2e-2);
-// below, the value is under 1e-22.  The sign of a zero result is kept, NaN
-// propagates; +inf gives NaN (inf * 0), which an f32 sum of 16-bit products
-// does not reach.
+// degree-10 polynomial for log2 Phi(-a) on [0, 10], its constant term the exact
+// -1, so that the error vanishes with x: 13 VALU instructions, one of them a
+// quarter-rate transcendental, 16 issue slots.  The coefficients are the
+// solution of a linear program: the smallest largest ratio of the error in
+// |x| q to the one 7.1.26 has in the same band of x, absolute and relative.
+// Evaluated in f32 it is the closer of the two in each band that
+// tests/test_gelu_fit.py lists: near zero 1.5e-7 relative (7.1.26: 6e-7),
+// 1.8e-7 absolute up to 3 and below the result's half ulp above (3.3e-7),
+// 7e-6 relative down to -3, 4e-4 to -5.5, 3.4e-3 to -10 (5e-5, 2.5e-3, 2e-2).
+// (Degree 8 cannot be that close in the tail, and an odd degree turns upwards
+// past the fit.)  With 7.1.26's P(t) e^{-a^2} it was 15 instructions, two of
+// them transcendentals, 21 slots, and the GELU bounds the stem's first level:
+// 300 chunks 357 -> 308 us with the rest of that kernel's changes, 15 chunks
+// 30.9 -> 19.1; fc1 over 3900 rows in bf16 34.3 -> 33.8.  (A degree-8 fit with a
+// free constant term took 33.3 and, at 15 chunks, 18.1, but was 6e-6 off near
+// zero: 0.7% of f16 results up to 0.1 rounded the other way.)  The sign of a zero
+// result is kept, NaN propagates; an infinite x, which a sum of bf16 products
+// or an infinite input can reach, gives NaN (inf * 0).
 __device__ __forceinline__ float gelu_erf(float x) {
   const float ax = fabsf(x);
-  float p = fmaf(ax, -6.02775501e-08f, 1.88221534e-07f);
-  p = fmaf(p, ax, 3.7997328e-05f);
-  p = fmaf(p, ax, -0.000805318821f);
-  p = fmaf(p, ax, 0.00817962456f);
-  p = fmaf(p, ax, -0.0535414778f);
-  p = fmaf(p, ax, -0.458688706f);
-  p = fmaf(p, ax, -1.15122461f);
-  const float q = __builtin_amdgcn_exp2f(fmaf(p, ax, -0.999991059f));
+  float p = fmaf(ax, -9.3436245e-09f, 3.7052223e-07f);
+  p = fmaf(p, ax, -6.002899e-06f);
+  p = fmaf(p, ax, 5.0021514e-05f);
+  p = fmaf(p, ax, -0.00019969424f);
+  p = fmaf(p, ax, -0.00014049842f);
+  p = fmaf(p, ax, 0.007088067f);
+  p = fmaf(p, ax, -0.052517902f);
+  p = fmaf(p, ax, -0.45920113f);
+  p = fmaf(p, ax, -1.1511059f);
+  const float q = __builtin_amdgcn_exp2f(fmaf(p, ax, -1.0f));
   // max(x, -0) as one v_max_f32: fmaxf adds a canonicalising v_max first,
   // which only matters for a NaN x, and a NaN x makes the FMA NaN anyway.
   // The instruction does not read %2 (p): that operand only orders the

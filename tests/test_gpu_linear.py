@@ -474,3 +474,30 @@ def test_silu_f16_packed_arithmetic_is_f32_then_f16(ctx, pkg, seed):
     from qwen3_aligner_wgpu_amd import host
 
     assert host.check_silu_f16x2(ctx, 1 << 23, seed) == 0
+
+
+def test_gelu_epilogue_rounds_like_the_exact_gelu(ctx, pkg, orc):
+    """GELU of every 16-bit value from 2^-10 to 10 in size (w picks one
+    element of the row, so the sum is the value itself).  Near zero an f32
+    evaluation with relative error d moves a result over one of f16's rounding
+    boundaries for a share d * 2^11 of the values at most: 3.1e-4 for the
+    1.5e-7 that gelu_erf keeps up to 0.1.  A bf16 result is within an ulp of the
+    exact one down to -7, where the tail's relative error is 8e-4 (ulp 4e-3)."""
+    from scipy.special import erfc
+    for dtype in (0, 1):
+        x = orc.h16_to_f32(np.arange(1 << 16, dtype=np.uint16), dtype).astype(np.float64)
+        keep = np.isfinite(x) & (np.abs(x) >= 2.0 ** -10) & (np.abs(x) <= 10.0)
+        bits, x = np.flatnonzero(keep).astype(np.uint16), x[keep]
+        a = np.zeros((len(bits), 8), np.uint16)
+        a[:, 0] = bits
+        w = _h16(orc, np.eye(1, 8).repeat(4, 0), dtype)
+        got = _run(ctx, pkg, dtype, a, w, np.zeros((len(bits), 4), np.uint16), flags=pkg.EPI_GELU)
+        assert (got == got[:, :1]).all()
+        exact = 0.5 * x * erfc(-x / np.sqrt(2.0))
+        if dtype == 0:
+            small = np.abs(x) <= 0.1
+            assert (got[small, 0] != exact[small].astype(np.float16).view(np.uint16)).mean() <= 5e-4
+        else:
+            part = x >= -7.0
+            v = orc.h16_to_f32(got[part, 0].copy(), dtype).astype(np.float64)
+            assert (np.abs(v - exact[part]) <= 2.0 ** (np.floor(np.log2(np.abs(exact[part]))) - 7)).all()
