@@ -226,6 +226,10 @@ qa::Plan plan_linear(const qa_linear_desc& d, int num_cus, size_t max_ws_floats 
   // for split-K partials, so batched calls are never split: the planner, not
   // the shape, must not decide whether a valid batched call can run.
   if (d.batch > 1) forced_splits = 1;
+  // ... but all of its problems' blocks share the chip, and are priced together
+  // (priced as one problem, 64 of 256 x 256 x 512 ran on 4096 32 x 32 tiles: 47
+  // us against 23 on 64 x 64).
+  const int64_t batch = std::max<int64_t>(1, d.batch);
 
   // every tile shape of the plain loader (TILE_256x160 is the conv loader's)
   int cands[] = {qa::TILE_128x128, qa::TILE_256x128, qa::TILE_128x256, qa::TILE_64x128,
@@ -256,7 +260,7 @@ qa::Plan plan_linear(const qa_linear_desc& d, int num_cus, size_t max_ws_floats 
       // partials that would not fit the caller's workspace bound (the
       // allocation-free entry point's scratch) rule a split count out
       if (splits > 1 && forced_splits <= 0 && (size_t)(splits * M * N) > max_ws_floats) break;
-      const int64_t units = tiles * splits;
+      const int64_t units = tiles * splits * batch;
       const int64_t rounds = (units + num_cus - 1) / num_cus;
       double cost = (double)rounds * (tile_fixed_us(cands[ci]) +
                                       stages_of(cands[ci], kchunk) * stage_us(cands[ci], units, num_cus));
