@@ -305,9 +305,11 @@ enum {
  *          [f][c], contiguous (the reference's permute,
  *          src/audio_encoder_gpu.rs:1795-1837, becomes a weight permutation).
  * Few output pixels with c_in > 1 split the contraction over f32 partials in
- * a buffer of the context that only convolutions use (never under stream
- * capture, where it may not grow and a replay would keep its address; without
- * memory for it the call runs unsplit).
+ * a 32 MiB buffer that the context allocates when it is created (without
+ * memory for it the calls run unsplit).  A call under stream capture is not
+ * split, so that its replays share nothing with the context's own calls: its
+ * sums run in another order than the same call's outside capture, and outputs
+ * may differ from that call's in the last place.
  * c_in = 1 (the mel input) or a multiple of 8 >= 64; c_out a multiple of 8
  * (<= 1024 when c_in = 1); every operand below 2 GiB. */
 typedef struct qa_conv_desc {

@@ -27,11 +27,11 @@ struct qa_ctx {
   int num_cus = 256;
   float* ws = nullptr;  // split-K partials
   size_t ws_floats = 0;
-  // Split convolutions' partials.  Not in `ws`: that one's address is kept by
-  // captured launches, and a convolution, which needs none for itself, must
-  // not be what replaces it under them.  No captured launch keeps this one's.
+  // Split convolutions' partials, kConvWsFloats of them or none: allocated with
+  // the context and never replaced, so that a convolution neither allocates
+  // nor waits.  Not in `ws`, whose address captured launches keep: a
+  // convolution must not be what replaces it under them.
   float* conv_ws = nullptr;
-  size_t conv_ws_floats = 0;
   float* scratch = nullptr;  // this device's copy of `scratch` (qa_linear_noalloc)
   // qa_prefetch_hint: bytes the projection after the next one reads; the next
   // projection launch takes it over and clears it
@@ -51,6 +51,10 @@ struct qa_ctx {
 // streams running at once) race on it.  Each split-K launch writes every
 // partial it later reads, so nothing needs clearing between calls.
 constexpr size_t kScratchFloats = (size_t)4 << 20;
+// The largest partials that plan_conv chooses for the audio tower's levels are
+// 7.7 M floats (4 or 5 chunks' second level, 19 chunks' third); a plan that
+// needs more than this is not taken.
+constexpr size_t kConvWsFloats = (size_t)8 << 20;
 static __device__ __align__(256) float scratch[kScratchFloats];
 
 namespace {
@@ -424,30 +428,6 @@ int ensure_workspace(qa_ctx* ctx, size_t floats) {
   return ok();
 }
 
-// The split convolutions' partials; false if there is no memory for them (the
-// caller then runs unsplit).  The thread's capture mode is relaxed meanwhile:
-// a convolution on this stream may run while another stream is captured, and
-// an allocation would break that capture.
-bool ensure_conv_workspace(qa_ctx* ctx, size_t floats) {
-  if (floats <= ctx->conv_ws_floats) return true;
-  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-  if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return false;
-  bool have = hipStreamSynchronize(ctx->stream) == hipSuccess;
-  if (have) {
-    if (ctx->conv_ws) (void)hipFree(ctx->conv_ws);
-    ctx->conv_ws = nullptr;
-    ctx->conv_ws_floats = 0;
-    have = hipMalloc(&ctx->conv_ws, floats * sizeof(float)) == hipSuccess;
-    if (have) ctx->conv_ws_floats = floats;
-    else {
-      ctx->conv_ws = nullptr;
-      (void)hipGetLastError();
-    }
-  }
-  (void)hipThreadExchangeStreamCaptureMode(&mode);
-  return have;
-}
-
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 float* g_scratch[kMaxDevices] = {};
@@ -577,6 +557,10 @@ int qa_ctx_create(int device, qa_ctx** out) {
   if (e != hipSuccess) {
     delete ctx;
     return hip_fail(e, "hipStreamCreateWithFlags");
+  }
+  if (hipMalloc(&ctx->conv_ws, kConvWsFloats * sizeof(float)) != hipSuccess) {
+    ctx->conv_ws = nullptr;  // convolutions run unsplit
+    (void)hipGetLastError();
   }
   *out = ctx;
   return ok();
@@ -915,11 +899,10 @@ int qa_conv2d_3x3s2(qa_ctx* ctx, const qa_conv_desc* d) {
     const hipError_t e = qa::launch_conv1((int)d->dtype, p, ctx->stream);
     return e == hipSuccess ? ok() : hip_fail(e, "qa_conv2d_3x3s2 launch");
   }
-  // A captured call is never split: its replays would go on using partials'
-  // memory that a later, larger call replaces, where the unsplit form uses none.
-  qa::Plan plan = plan_conv(M, d->c_out, K, gelu, ctx->num_cus, capturing(ctx) ? 0 : SIZE_MAX);
-  if (plan.splits > 1 && !ensure_conv_workspace(ctx, plan.ws_floats))
-    plan = plan_conv(M, d->c_out, K, gelu, ctx->num_cus, 0);
+  // A captured call is not split: its replays may run on another stream, next to
+  // a convolution on this one, and would share the partials with it.
+  const bool split = ctx->conv_ws && !capturing(ctx);
+  const qa::Plan plan = plan_conv(M, d->c_out, K, gelu, ctx->num_cus, split ? kConvWsFloats : 0);
   qa::GemmParams p{};
   p.ws = ctx->conv_ws;
   p.a = (const uint16_t*)d->x;

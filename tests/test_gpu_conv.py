@@ -94,15 +94,14 @@ def test_conv_tiles_and_no_activation(ctx, pkg, orc, monkeypatch, tile):
 
 
 @pytest.mark.parametrize("dtype", [F16, BF16], ids=["f16", "bf16"])
-@pytest.mark.parametrize("tile,splits", [("0", "2"), ("1", "3"), ("2", "5"), ("6", "2"), ("8", "9"), ("", "")])
+@pytest.mark.parametrize("tile,splits", [("0", "2"), ("1", "3"), ("2", "5"), ("6", "2"), ("8", "9")])
 @pytest.mark.parametrize("tmajor", [False, True], ids=["rows_hw", "rows_wh"])
 def test_conv_split_k(ctx, pkg, orc, monkeypatch, dtype, tile, splits, tmajor):
     """K split over f32 partials and the reduce kernel, on every tile shape
-    (taps and channels of a split start inside a tap; 14 stages, uneven splits),
-    and the planner's own choice at this size: bias, GELU, both row orders."""
-    if tile:
-        monkeypatch.setenv("QA_TILE", tile)
-        monkeypatch.setenv("QA_SPLITS", splits)
+    (taps and channels of a split start inside a tap; 14 stages, uneven splits):
+    bias, GELU, both row orders."""
+    monkeypatch.setenv("QA_TILE", tile)
+    monkeypatch.setenv("QA_SPLITS", splits)
     x, wt, bias = _case(orc, dtype, 2, 20, 18, 96, 200, 7)
     flags = pkg.QA_CONV_GELU | (pkg.QA_CONV_TOKEN_MAJOR if tmajor else 0)
     got = _conv_gpu(ctx, pkg, dtype, x, wt, bias, 200, flags)
@@ -111,30 +110,81 @@ def test_conv_split_k(ctx, pkg, orc, monkeypatch, dtype, tile, splits, tmajor):
     assert np.array_equal(got, _conv_gpu(ctx, pkg, dtype, x, wt, bias, 200, flags))
 
 
-def test_conv_captured_without_workspace(pkg, orc):
-    """On a fresh context a captured convolution runs unsplit (no workspace):
-    every replay within one ulp, also after eager calls grew the workspace."""
+SHORT = (2, 32, 25, 480, 480)  # the third level of two chunks: 16 tiles of 128 x 128, which the planner splits in six
+
+
+def _short(orc, dtype):
+    b, h, w, c_in, c_out = SHORT
+    return _case(orc, dtype, b, h, w, c_in, c_out, 13)
+
+
+def _conv_desc(pkg, dtype, x, wt, bias, y):
+    b, h, w, c_in, c_out = SHORT
+    return pkg.ConvDesc(dtype=dtype, flags=pkg.QA_CONV_GELU, batch=b, h=h, w=w, c_in=c_in, c_out=c_out,
+                        x=int(x), weight=int(wt), bias=int(bias), y=int(y))
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("tmajor", [False, True], ids=["rows_hw", "rows_wh"])
+def test_conv_planner_splits_short_clips(ctx, pkg, orc, monkeypatch, dtype, tmajor):
+    """The planner's own split: other bits than the unsplit call's (sums in
+    another order), the same in each call, and right."""
+    x, wt, bias = _short(orc, dtype)
+    flags = pkg.QA_CONV_GELU | (pkg.QA_CONV_TOKEN_MAJOR if tmajor else 0)
+    got = _conv_gpu(ctx, pkg, dtype, x, wt, bias, SHORT[-1], flags)
+    assert_parity(got, orc.conv3x3s2(dtype, x, wt, bias, gelu=True, token_major=tmajor), orc, dtype, ulp_tol=1)
+    assert np.array_equal(got, _conv_gpu(ctx, pkg, dtype, x, wt, bias, SHORT[-1], flags))
+    monkeypatch.setenv("QA_SPLITS", "1")
+    assert not np.array_equal(got, _conv_gpu(ctx, pkg, dtype, x, wt, bias, SHORT[-1], flags))
+
+
+def test_conv_captured_runs_unsplit(pkg, orc, monkeypatch):
+    """A captured convolution that would be split when eager runs unsplit: every
+    replay has the unsplit call's bits, also with eager, split calls between."""
     from hipgraph import Capture
-    x, wt, bias = _case(orc, F16, 2, 20, 18, 96, 200, 7)
+    x, wt, bias = _short(orc, F16)
     want = orc.conv3x3s2(F16, x, wt, bias, gelu=True)
     with pkg.Context(0) as ctx:
         dx, dw, db = ctx.to_device(x), ctx.to_device(wt), ctx.to_device(bias)
         dy, dz = ctx.alloc(want.size * 2), ctx.alloc(want.size * 2)
-
-        def run(y):
-            ctx.conv2d_3x3s2(pkg.ConvDesc(dtype=F16, flags=pkg.QA_CONV_GELU, batch=2, h=20, w=18, c_in=96, c_out=200,
-                                          x=int(dx), weight=int(dw), bias=int(db), y=int(y)))
-
+        monkeypatch.setenv("QA_SPLITS", "1")
+        ctx.conv2d_3x3s2(_conv_desc(pkg, F16, dx, dw, db, dz))
+        unsplit = ctx.download(dz, want.shape)
+        monkeypatch.delenv("QA_SPLITS")
         with Capture(ctx.stream) as cap:
-            run(dy)
+            ctx.conv2d_3x3s2(_conv_desc(pkg, F16, dx, dw, db, dy))
         for _ in range(3):
             ctx.upload(dy, np.zeros(want.shape, np.uint16))
             cap.replay()
-            assert_parity(ctx.download(dy, want.shape), want, orc, F16, ulp_tol=1)
-            run(dz)  # eager, split
+            assert np.array_equal(ctx.download(dy, want.shape), unsplit)
+            ctx.conv2d_3x3s2(_conv_desc(pkg, F16, dx, dw, db, dz))
             ctx.sync()
-        assert_parity(ctx.download(dz, want.shape), want, orc, F16, ulp_tol=1)
+        eager = ctx.download(dz, want.shape)
+        assert not np.array_equal(eager, unsplit)
+        assert_parity(unsplit, want, orc, F16, ulp_tol=1)
+        assert_parity(eager, want, orc, F16, ulp_tol=1)
         cap.close()
+
+
+def test_conv_allocates_nothing(ctx, pkg):
+    """The first split convolution of a context takes no device memory (3 x 2080
+    x 480 partials, 12 MB, for ten chunks' third level): the buffer is the
+    context's from its creation."""
+    import torch
+    b, h, w, c_in, c_out = SHORT
+    x, wt, bias = ctx.alloc(5 * b * h * w * c_in * 2), ctx.alloc(c_out * 9 * c_in * 2), ctx.alloc(c_out * 2)
+    y = ctx.alloc(5 * b * 16 * 13 * c_out * 2)
+    desc = _conv_desc(pkg, F16, x, wt, bias, y)
+    desc.batch = 5 * b
+    ctx.conv2d_3x3s2(desc)  # loads the kernels' code
+    ctx.sync()
+    with pkg.Context(0) as fresh:
+        before = torch.cuda.mem_get_info()[0]
+        fresh.conv2d_3x3s2(desc)
+        fresh.sync()
+        assert torch.cuda.mem_get_info()[0] == before
+    for buf in (x, wt, bias, y):
+        buf.free()
 
 
 def test_conv_leaves_captured_workspace(pkg, orc, monkeypatch):
