@@ -9,6 +9,11 @@
 
 #include "qa.h"
 
+// libqa.so, for this file alone: whether convolutions recorded on the
+// context's captured stream split their contraction as eager ones do.  Only
+// for a graph whose replays stay in order with the context's own work.
+extern "C" void qa_ctx_split_captured_convs(qa_ctx* ctx, int on);
+
 namespace qa_host {
 
 inline int timing_status(hipError_t e) { return e == hipSuccess ? QA_OK : QA_EDEVICE; }
@@ -19,7 +24,8 @@ inline int timing_status(hipError_t e) { return e == hipSuccess ? QA_OK : QA_EDE
 // of a step sizes the context's workspace, which cannot grow under capture).
 // Warm-up steps taken eagerly instead, with the graph launched once before
 // the timed replays, left the first timed run of a process ~3.5% slower than
-// a second one.
+// a second one.  The graph is replayed on the context's stream alone, so its
+// convolutions are the eager step's.
 template <class Step>
 int time_steps(qa_ctx* ctx, int warmup, int steps, int use_graph, Step&& step, double* ms,
                double* wall_ms = nullptr) {
@@ -32,7 +38,9 @@ int time_steps(qa_ctx* ctx, int warmup, int steps, int use_graph, Step&& step, d
   hipGraph_t graph = nullptr;
   if (use_graph) {
     if (hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) != hipSuccess) return QA_EDEVICE;
+    qa_ctx_split_captured_convs(ctx, 1);
     const int rc = step();
+    qa_ctx_split_captured_convs(ctx, 0);
     const hipError_t ec = hipStreamEndCapture(s, &graph);
     if (rc) return rc;
     if (ec != hipSuccess) return QA_EDEVICE;

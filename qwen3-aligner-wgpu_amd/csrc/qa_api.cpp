@@ -32,6 +32,7 @@ struct qa_ctx {
   // nor waits.  Not in `ws`, whose address captured launches keep: a
   // convolution must not be what replaces it under them.
   float* conv_ws = nullptr;
+  bool conv_split_captured = false;  // see qa_ctx_split_captured_convs
   float* scratch = nullptr;  // this device's copy of `scratch` (qa_linear_noalloc)
   // qa_prefetch_hint: bytes the projection after the next one reads; the next
   // projection launch takes it over and clears it
@@ -566,6 +567,8 @@ int qa_ctx_create(int device, qa_ctx** out) {
   return ok();
 }
 
+void qa_ctx_split_captured_convs(qa_ctx* ctx, int on) { ctx->conv_split_captured = on != 0; }
+
 int qa_ctx_destroy(qa_ctx* ctx) {
   if (!ctx) return ok();
   (void)hipSetDevice(ctx->device);
@@ -901,7 +904,7 @@ int qa_conv2d_3x3s2(qa_ctx* ctx, const qa_conv_desc* d) {
   }
   // A captured call is not split: its replays may run on another stream, next to
   // a convolution on this one, and would share the partials with it.
-  const bool split = ctx->conv_ws && !capturing(ctx);
+  const bool split = ctx->conv_ws && (ctx->conv_split_captured || !capturing(ctx));
   const qa::Plan plan = plan_conv(M, d->c_out, K, gelu, ctx->num_cus, split ? kConvWsFloats : 0);
   qa::GemmParams p{};
   p.ws = ctx->conv_ws;

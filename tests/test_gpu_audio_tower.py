@@ -138,3 +138,22 @@ def test_audio_tower_chain(ctx, pkg, orc, dtype, n_chunks, tail):
     rel_rms = np.sqrt(((g - r) ** 2).mean() / (r ** 2).mean())
     assert mae <= 1e-3 * (1 if dtype == F16 else 8), mae
     assert rel_rms <= ulp, rel_rms
+
+
+def test_timed_graph_runs_the_eager_step(ctx, pkg, orc):
+    """time(use_graph) leaves what forward() computes, bit for bit, also for a
+    short clip, whose convolutions are split: what it times is that step."""
+    n_chunks = 2
+    w = _weights(orc, F16, 1, 21)
+    enc = _build(ctx, F16, w, n_chunks)
+    try:
+        n = enc.tokens(n_chunks, 0)
+        enc.set_mel(_mel(orc, F16, n_chunks, 0, 22))
+        enc.forward(n_chunks, 0)
+        want = [enc.read(k, r).copy() for k, r in (("conv3", n_chunks * 13), ("out", n))]
+        enc.time(n_chunks, 0, 2, 3, use_graph=True)
+        got = [enc.read(k, r).copy() for k, r in (("conv3", n_chunks * 13), ("out", n))]
+    finally:
+        enc.close()
+    for g, e in zip(got, want):
+        assert np.array_equal(g, e)
