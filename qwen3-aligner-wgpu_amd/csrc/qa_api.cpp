@@ -849,6 +849,7 @@ int qa_attention_prefill(qa_ctx* ctx, const qa_attention_desc* d) {
   p.nqh = d->nqh;
   p.nkvh = d->nkvh;
   p.hd = d->hd;
+  p.num_cus = ctx->num_cus;
   p.scale = 1.0f / sqrtf((float)d->hd);
   const hipError_t e = qa::launch_attention((int)d->dtype, p, (d->flags & QA_ATTN_P16) != 0, ctx->stream);
   return e == hipSuccess ? ok() : hip_fail(e, "qa_attention_prefill launch");

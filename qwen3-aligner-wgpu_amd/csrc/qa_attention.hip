@@ -621,12 +621,7 @@ hipError_t launch_ps(const AttnParams& p, hipStream_t s) {
   const int rep = p.nqh / p.nkvh;
   if (rep == 1) return launch_shape<DT, 1, PS, 2, 2, 2>(p, s);
   if (rep != 2) return hipErrorInvalidValue;  // rejected by qa_attention_prefill's validation
-  // 32-row blocks while the 64-row ones would not fill the 256 CUs, unless
-  // they need a second round of blocks about as long as the first (the
-  // figures are at the top of the file)
-  const bool one_round = (p.rows + 31) / 32 * p.nkvh <= 256;
-  if (one_round || ((p.rows + 63) / 64 * p.nkvh <= 256 && 2 * p.q0 < 3 * p.rows))
-    return launch_shape<DT, 2, PS, 1, 4, 1>(p, s);
+  if (attention_32_row_blocks(p)) return launch_shape<DT, 2, PS, 1, 4, 1>(p, s);
   return launch_shape<DT, 2, PS, 2, 2, 2>(p, s);
 }
 

@@ -259,8 +259,17 @@ struct AttnParams {
   uint16_t* out;
   int64_t rows, cap, q0, ldo;
   int nqh, nkvh, hd;
+  int num_cus;
   float scale;
 };
+// Whether attention takes blocks of 32 query rows (two q heads per kv head): as
+// long as those of 64 would not fill the CUs, unless a second round of 32-row
+// blocks is about as long as the first.  The figures are at the top of
+// qa_attention.hip.
+inline bool attention_32_row_blocks(const AttnParams& p) {
+  const bool one_round = (p.rows + 31) / 32 * p.nkvh <= p.num_cus;
+  return one_round || ((p.rows + 63) / 64 * p.nkvh <= p.num_cus && 2 * p.q0 < 3 * p.rows);
+}
 // Audio tower ops (qa_audio_ops.hip).
 struct LnParams {
   const uint16_t* x;

@@ -1,5 +1,5 @@
-"""The projection planner (plan_linear in csrc/qa_api.cpp) on the CPU: qa_api.cpp
-compiled into a small library of the test's own that returns its plans."""
+"""The rules that choose a launch's shape, on the CPU: csrc/qa_api.cpp (plan_linear)
+and qa_internal.h compiled into a small library of the test's own."""
 from __future__ import annotations
 
 import ctypes
@@ -25,6 +25,14 @@ extern "C" void test_plan_linear(uint32_t flags, int64_t m, int64_t n, int64_t k
   out[1] = p.splits;
   out[2] = p.tiles_m;
   out[3] = p.tiles_n;
+}
+extern "C" int test_attention_32(int64_t rows, int64_t q0, int nkvh, int cus) {
+  qa::AttnParams p{};
+  p.rows = rows;
+  p.q0 = q0;
+  p.nkvh = nkvh;
+  p.num_cus = cus;
+  return qa::attention_32_row_blocks(p);
 }
 """
 
@@ -62,3 +70,17 @@ def test_batch_is_priced_as_a_whole(planner, m, n, k, batch):
     if one[1] == 1:
         assert got[0] == one[0]
     assert _linear(planner, m, n, k, 0) == _linear(planner, m, n, k, 1)
+
+
+@pytest.mark.parametrize("cus", [32, 64, 256])
+def test_attention_shape_counts_the_devices_cus(planner, cus):
+    """32-row blocks up to one 64-row block per CU of the device in use (a
+    partition of the chip has fewer than 256), or, behind a long past, up to
+    one 32-row block per CU."""
+    def blocks32(rows, q0):
+        i64 = ctypes.c_int64
+        return bool(planner.test_attention_32(i64(rows), i64(q0), 8, cus))
+
+    full = cus // 8  # blocks of one kv head in a round
+    assert blocks32(64 * full, 0) and not blocks32(64 * full + 1, 0)
+    assert blocks32(32 * full, 10 * 32 * full) and not blocks32(32 * full + 1, 2 * 32 * full)
