@@ -142,12 +142,13 @@ __global__ void __launch_bounds__(256) conv1_kernel(const Conv1Params p, int gro
 hipError_t launch_conv1(int dtype, const Conv1Params& p, hipStream_t s) {
   if (p.c_out > kMaxCout) return hipErrorInvalidValue;  // rejected by validation
   const unsigned blocks = (unsigned)((p.M + kPix - 1) / kPix);
-  // All of a pixel's channels in one block where that gives the chip several
-  // blocks per CU in each of a few rounds; else groups of five tiles (160
-  // channels), so that the last round of a short clip is not mostly idle:
-  // 15 chunks (375 pixel blocks) 30.9 -> 19.1 us with all of this file's changes;
-  // one group at 300 chunks (7500) 357 -> 308 us.
-  const int tiles = (p.c_out + 31) / 32, group = blocks >= 2048 ? tiles : 5;
+  // Groups of five tiles (160 channels) per block, so that a short clip's last
+  // round is not mostly idle; all of a pixel's channels in one block for the
+  // longest clips, whose rows are then written whole.  480 channels, f16, groups of 5 against one of 15, us by pixel blocks:
+  // 375 18.9 / 24.0, 1000 38.5 / 38.4, 2050 73 / 74, 3000 111 / 118, 3750 141 / 171,
+  // 5000 186 / 221, 6250 294 / 263, 7500 384 / 308, 10000 555 / 398.  (Groups of one
+  // to three are 10-35% faster up to 125, 2-8% slower from 500 on.)
+  const int tiles = (p.c_out + 31) / 32, group = blocks >= 5632 ? tiles : 5;
   const dim3 g(blocks, (unsigned)((tiles + group - 1) / group)), t(256);
   if (dtype == QA_BF16) {
     if (p.gelu) hipLaunchKernelGGL((conv1_kernel<QA_BF16, true>), g, t, 0, s, p, group);

@@ -361,9 +361,12 @@ hipError_t launch_timestamp_head(int dtype, const HeadParams& p, hipStream_t s) 
       p.labels * p.n * 4 < kSpan) {
     const int64_t rb = (p.rows + 31) / 32;
     auto blocks = [&](int64_t lb) { return dim3((unsigned)(((p.labels + lb - 1) / lb + 7) / 8 * 8 * rb)); };
-    // 64 labels per block read the rows half as often; 32 where those blocks
-    // would leave half the CUs idle (one row block, up to 32 slots, of 5000
-    // labels: 79 blocks).  At 78 rows 64 labels take 17.0 us, 32 take 20.1.
+    // 64 labels per block read the rows half as often; 32 as long as the blocks
+    // then make one round (up to 128 blocks of 64: up to 32 slots of 5000
+    // labels).  The whole head with 32 / 64 labels a block, us: 5000 labels, 32
+    // rows (79 blocks of 64) 17.5 / 21.7, 33 (158) 25.0 / 21.8, 78 (237) 25.5 /
+    // 22.4, 240 (632) 49.0 / 43.5; 2500 labels, 96 rows (120) 16.9 / 21.2, 97
+    // (160) 24.1 / 22.1; 10000 labels, 32 rows (157) 26.8 / 24.2.
     if ((p.labels + 63) / 64 * rb > 128)
       hipLaunchKernelGGL(head_logits_kernel<2>, blocks(64), t8, 0, s, p);
     else

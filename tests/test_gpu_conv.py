@@ -82,6 +82,18 @@ def test_conv(ctx, pkg, orc, dtype, b, h, w, c_in, c_out, tmajor):
     assert_parity(got, want, orc, dtype, ulp_tol=1)
 
 
+@pytest.mark.parametrize("batch", [900, 901])
+def test_conv1_groups(ctx, pkg, orc, batch):
+    """Level 1 in two channel groups (5625 blocks of 128 pixels) and with all six
+    channel tiles in one block (5632, the last a quarter full): the bits of two
+    images' own call, in every place."""
+    x, wt, bias = _case(orc, F16, 2, 64, 50, 1, 168, 17)
+    want = _conv_gpu(ctx, pkg, F16, x, wt, bias, 168, pkg.QA_CONV_GELU).reshape(2, -1)
+    assert_parity(want.reshape(-1, 168), orc.conv3x3s2(F16, x, wt, bias, gelu=True), orc, F16, ulp_tol=1)
+    got = _conv_gpu(ctx, pkg, F16, x[np.arange(batch) % 2], wt, bias, 168, pkg.QA_CONV_GELU).reshape(batch, -1)
+    assert (got[0::2] == want[0]).all() and (got[1::2] == want[1]).all()
+
+
 @pytest.mark.parametrize("tile", ["0", "1", "2", "6", "8"],
                          ids=["128x128", "256x128", "128x256", "256x256", "256x160"])
 def test_conv_tiles_and_no_activation(ctx, pkg, orc, monkeypatch, tile):
