@@ -21,10 +21,11 @@
 //    groups hold one K and one V tile each (NB = 1: 128 KB), refilled during
 //    the VALU phase, longer than the L2 takes to answer; with two of each of
 //    half the keys a step's fixed costs double (1024 rows: 20.1 us).
-//    Measured, f16, RG = 2 -> RG = 1: 61 rows 8.3 -> 7.1 us, 323 rows 12.9 ->
-//    10.5, 1024 rows 25.2 -> 17.8, 2048 rows (256 blocks of 64) 42.6 -> 36.1,
-//    2200 rows (280) 46.0 -> 48.3; 771 rows from position 1536 with 16-bit
-//    probabilities 38.8 -> 24.6.  Hence the line at 256 blocks of 64 rows.
+//    Measured, f16, repeated launches, RG = 2 -> RG = 1: 61 rows 7.7 -> 6.7 us,
+//    323 rows 12.9 -> 10.4, 1024 rows 24.5 -> 16.9, 2048 rows (256 blocks of 64)
+//    41.9 -> 36.3, 2200 rows (280) 46.0 -> 48.3; 771 rows from position 1536 with
+//    16-bit probabilities 38.6 -> 24.4.  Hence the line at one block of 64 rows
+//    per CU.
 //    Behind a long past the blocks are all about equally long, and 257 to 512
 //    of 32 rows take two full rounds: 8 kv heads, 1200 rows from position
 //    1000 43.0 -> 40.3 us, 1500 51.1 -> 50.6, 2000 58.8 -> 60.9, 4000 91 ->

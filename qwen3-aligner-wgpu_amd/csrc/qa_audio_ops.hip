@@ -188,14 +188,14 @@ __global__ void __launch_bounds__(256) add_table_kernel(const TableAddParams p) 
 // stored in the order the score layout holds the keys: within each aligned
 // group of 16 keys, 0-3, 8-11, 4-7, 12-15 (bits 2 and 3 swapped).
 //
-// Bound by latency: up to about 15 windows of 16 heads every block has a CU of
+// Bound by latency: up to 18 windows of 14 heads every block has a CU of
 // its own, and its time is one trip to memory, the LDS
 // traffic around one barrier and the launch.  So every load of the block is issued before the
 // first LDS store waits for one (K, V and Q one after another were three
 // trips), on rows clamped to the window so that no load sits behind a branch,
 // and each 32-key tile's O products follow its probabilities while the next
-// tile's exponentials run.  16 heads, windows of 104, f16: 26 tokens 5.4 us
-// with the loads in turn, 5.1 now; 390 tokens 6.3, 6.0; 3900 tokens 11.2, 10.9.
+// tile's exponentials run.  14 heads, windows of 104, f16: 26 tokens 5.3 us
+// with the loads in turn, 5.05 now; 390 tokens 6.3, 6.0; 3900 tokens 11.2, 10.65.
 constexpr int WA_HD = 64, WA_MAXW = 128;
 
 

@@ -44,7 +44,19 @@ def _draw(seed):
 
 @pytest.mark.parametrize("seed", range(CASES))
 def test_random_linear(ctx, pkg, orc, seed):
-    rng, dtype, m, n, k, nout, kind, (pa, pb, pc), tile, splits = _draw(seed)
+    _check(ctx, pkg, orc, *_draw(seed))
+
+
+@pytest.mark.parametrize("tile", [10, 11])
+@pytest.mark.parametrize("seed", range(301, 317))
+def test_random_linear_32_row_tiles(ctx, pkg, orc, seed, tile):
+    """The same over the 32-row tiles, unsplit to split in three (the 16 seeds hold
+    every epilogue twice or more; 11 has no SiLU.up: 10 takes it)."""
+    _check(ctx, pkg, orc, *_draw(seed)[:-2], tile, 1 + seed % 3)
+
+
+def _check(ctx, pkg, orc, rng, dtype, m, n, k, nout, kind, pads, tile, splits):
+    pa, pb, pc = pads
     lda, ldb, ldc = k + pa, k + pb, nout + pc
     a = _h16(orc, rng.standard_normal((m, k)), dtype)
     w = _h16(orc, 0.05 * rng.standard_normal((n, k)), dtype)
