@@ -73,6 +73,34 @@ def test_no_band_is_further_off_than_7_1_26(lo, hi, sign):
     assert got[0] <= max(bar[0], half_ulp * 1.05) and got[1] <= max(bar[1], half_ulp * 1.05 / lo), (got, bar)
 
 
+def test_coefficients_solve_the_fit():
+    """How they were found: the linear program for the degree-10 polynomial, its
+    constant term -1, with the smallest largest ratio of the error in |x| q to
+    7.1.26's largest in the same band (the smaller of its absolute and its
+    relative one, 0.7 of that past 4, at least 3e-9 x below 1, where f32 rounds
+    more).  Its optimum is 0.24; rounded to f32 the coefficients keep 0.34."""
+    from scipy.optimize import linprog
+    from scipy.special import log_ndtr, ndtr
+    a = np.concatenate([np.geomspace(1e-3, 0.2, 300), np.linspace(0.2, 10, 1500)])
+    q = ndtr(-a)
+    t = 1 / (1 + 0.3275911 * a / np.sqrt(2))
+    old = 0.5 * t * np.exp(-a * a / 2) * np.polyval([1.061405429, -1.453152027, 1.421413741, -0.284496736, 0.254829592], t)
+    bar = np.empty_like(a)
+    for lo, hi in zip(BANDS[1:], BANDS[2:-1] + [11]):
+        m = (a >= lo) & (a < hi)
+        bar[m] = np.minimum((a * np.abs(old - q))[m].max(), (a * q)[m] * np.abs(old / q - 1)[m].max())
+    bar = np.maximum(bar, np.where(a < 1, 3e-9 * a, 0)) * np.where(a > 4, 0.7, 1)
+    w = a * q * np.log(2) / bar
+    scale = 10.0 ** np.arange(1, 11)  # of the unknowns, for the solver
+    rows = w[:, None] * np.stack([a ** k for k in range(1, 11)], 1) / scale
+    rhs = w * (log_ndtr(-a) / np.log(2) + 1)
+    one = np.ones((len(a), 1))
+    best = linprog(np.r_[np.zeros(10), 1], A_ub=np.block([[rows, -one], [-rows, -one]]), b_ub=np.r_[rhs, -rhs],
+                   bounds=[(None, None)] * 10 + [(0, None)], method="highs").x[-1]
+    mine = np.array(_coefficients(), np.float64)[::-1][1:]
+    assert np.abs(rows @ (mine * scale) - rhs).max() <= 0.35 and best < 0.25
+
+
 def test_falls_past_the_fit():
     """Past 10 the polynomial keeps falling (its leading coefficient is
     negative), to an exponent that gives a zero: no value comes back up."""
