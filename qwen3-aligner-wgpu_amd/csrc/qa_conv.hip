@@ -146,8 +146,8 @@ hipError_t launch_conv1(int dtype, const Conv1Params& p, hipStream_t s) {
   // round is not mostly idle; all of a pixel's channels in one block for the
   // longest clips, whose rows are then written whole.  480 channels, f16, groups of 5 against one of 15, us by pixel blocks:
   // 375 18.9 / 24.0, 1000 38.5 / 38.4, 2050 73 / 74, 3000 111 / 118, 3750 141 / 171,
-  // 5000 186 / 221, 6250 294 / 263, 7500 384 / 308, 10000 555 / 398.  (Groups of one
-  // to three are 10-35% faster up to 125, 2-8% slower from 500 on.)
+  // 5000 186 / 221, 6250 294 / 263, 7500 384 / 308, 10000 555 / 398.  (Groups of two
+  // are 14-31% faster up to 125 and 6-12% slower from 500 on.)
   const int tiles = (p.c_out + 31) / 32, group = blocks >= 5632 ? tiles : 5;
   const dim3 g(blocks, (unsigned)((tiles + group - 1) / group)), t(256);
   if (dtype == QA_BF16) {
